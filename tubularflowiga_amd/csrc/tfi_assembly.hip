@@ -21,6 +21,7 @@
 //     read-modify-write: elements of one colour share no node, colours run
 //     in order, so every block sum has a fixed order (no atomics).
 #include "tfi_internal.hpp"
+#include "tfi_point.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -34,16 +35,6 @@ constexpr size_t kLdsLimit = 160*1024;  // gfx950 LDS per workgroup
 constexpr int kQd = 56;       // per-point record in LDS
 constexpr int kBasisRec = 7;  // N, dN/dx, dN/dy, dN/dz, lap N, u.grad N, w.grad N (w = u + u')
 static_assert(kMaxBasis % 2 == 0, "the connectivity ints fill whole doubles of the LDS carve-up");
-
-__constant__ double kGp[4] = {0.06943184420297371, 0.33000947820757187, 0.6699905217924281, 0.9305681557970262};
-
-__device__ inline void Bern3(double x, double b[4], double db[4], double d2b[4])
-{
-	const double y = 1.0 - x;
-	b[0] = y*y*y; b[1] = 3.0*y*y*x; b[2] = 3.0*y*x*x; b[3] = x*x*x;
-	db[0] = -3.0*y*y; db[1] = 3.0 - 12.0*x + 9.0*x*x; db[2] = 3.0*(2.0 - 3.0*x)*x; db[3] = 3.0*x*x;
-	d2b[0] = 6.0*y; d2b[1] = -12.0 + 18.0*x; d2b[2] = 6.0 - 18.0*x; d2b[3] = 6.0*x;
-}
 
 constexpr int kTableRec = 5;  // N, dN/dx, dN/dy, dN/dz, lap N
 constexpr int kPointGeom = 10;  // geometry fields the point record reads: measure, J^-1
@@ -83,86 +74,6 @@ __device__ inline void EvalBasis(const double* __restrict__ c, const double* __r
 	out[4] = h00*gq[10*kQ] + h11*gq[11*kQ] + h22*gq[12*kQ]
 		+ 2.0*(h01*gq[13*kQ] + h02*gq[14*kQ] + h12*gq[15*kQ])
 		+ g0*gq[16*kQ] + g1*gq[17*kQ] + g2*gq[18*kQ];
-}
-
-// Per-point record from the field sums s (u, p, grad u, grad p, lap u, u_prev
-// at the point; 22 values) and the point's geometry record gq (fields 0..9:
-// measure and J^-1, field stride kGs): r[0] measure, r[1..2] tau_M, tau_C, r[3..5] u, r[6..8] rho (du/dt +
-// w.grad u), r[9..17] stress rows, r[18] div u, r[19..21] u', r[22..24] w =
-// u + u', r[25..33] grad u and, with exact_tangent, r[34..54] the
-// linearisation of u' (K, R, c1) the consistent tangent needs.
-template <int kGs>
-__device__ inline void PointRecord(const double* __restrict__ s, const double* __restrict__ gq, double rho, double mu,
-	double nu, double dt, bool exact_tangent, double* __restrict__ r)
-{
-	double inv[3][3];
-	for (int a = 0; a < 3; ++a)
-		for (int x = 0; x < 3; ++x) inv[a][x] = gq[(1 + 3*a + x)*kGs];
-	const double u[3] = {s[0], s[1], s[2]};
-	const double p = s[3];
-	double grad[4][3];
-	for (int f = 0; f < 4; ++f)
-		for (int d = 0; d < 3; ++d) grad[f][d] = s[4 + 3*f + d];
-	double dudt[3];
-	for (int c = 0; c < 3; ++c) dudt[c] = dt > 0.0 ? (u[c] - s[19 + c])/dt : 0.0;
-	double G[3][3] = {}, gv[3] = {};
-	for (int i = 0; i < 3; ++i)
-		for (int j = 0; j < 3; ++j) {
-			for (int k = 0; k < 3; ++k) G[i][j] += inv[k][i]*inv[k][j];
-			gv[i] += inv[j][i];
-		}
-	double GG = 0.0, gg = 0.0, uGu = 0.0;
-	for (int i = 0; i < 3; ++i) {
-		gg += gv[i]*gv[i];
-		for (int j = 0; j < 3; ++j) {
-			GG += G[i][j]*G[i][j];
-			uGu += u[i]*G[i][j]*u[j];
-		}
-	}
-	const double temporal = dt > 0.0 ? 4.0/(dt*dt) : 0.0;
-	const double tau_m = 1.0/sqrt(temporal + uGu + (1.0/12.0)*nu*nu*GG);
-	const double tau_c = 1.0/(tau_m*gg);
-	double fu[3];
-	for (int c = 0; c < 3; ++c) {
-		const double conv = u[0]*grad[c][0] + u[1]*grad[c][1] + u[2]*grad[c][2];
-		fu[c] = -tau_m*(dudt[c] + conv + grad[3][c]/rho - nu*s[16 + c]);
-	}
-	const double div = grad[0][0] + grad[1][1] + grad[2][2];
-	const double fp = -rho*tau_c*div;
-	r[0] = gq[0];
-	r[1] = tau_m;
-	r[2] = tau_c;
-	for (int c = 0; c < 3; ++c) r[3 + c] = u[c];
-	const double w[3] = {u[0] + fu[0], u[1] + fu[1], u[2] + fu[2]};
-	for (int c = 0; c < 3; ++c) {
-		r[6 + c] = rho*(dudt[c] + w[0]*grad[c][0] + w[1]*grad[c][1] + w[2]*grad[c][2]);
-		for (int d = 0; d < 3; ++d)
-			r[9 + 3*c + d] = mu*(grad[c][d] + grad[d][c]) - rho*fu[c]*w[d] - (c == d ? p + fp : 0.0);
-	}
-	r[18] = div;
-	for (int c = 0; c < 3; ++c) r[19 + c] = fu[c];
-	for (int c = 0; c < 3; ++c) r[22 + c] = w[c];
-	for (int c = 0; c < 3; ++c)
-		for (int d = 0; d < 3; ++d) r[25 + 3*c + d] = grad[c][d];
-	if (exact_tangent) {
-		// d(u')/d(u_f) = N_b K[.][f] - delta tau_M s_b with
-		// K_cf = tau_M^3 strong_c (G u)_f - tau_M du_c/dx_f, and
-		// R = grad u + grad u K, c1_f = rho tau_C tau_M^2 div (G u)_f.
-		double Gu[3];
-		for (int i = 0; i < 3; ++i) Gu[i] = G[i][0]*u[0] + G[i][1]*u[1] + G[i][2]*u[2];
-		const double tm3 = tau_m*tau_m*tau_m;
-		double K[3][3];
-		for (int c = 0; c < 3; ++c) {
-			const double strong = -fu[c]/tau_m;
-			for (int f = 0; f < 3; ++f) K[c][f] = tm3*strong*Gu[f] - tau_m*grad[c][f];
-		}
-		for (int c = 0; c < 3; ++c)
-			for (int f = 0; f < 3; ++f) {
-				r[34 + 3*c + f] = K[c][f];
-				r[43 + 3*c + f] = grad[c][f] + grad[c][0]*K[0][f] + grad[c][1]*K[1][f] + grad[c][2]*K[2][f];
-			}
-		for (int f = 0; f < 3; ++f) r[52 + f] = rho*tau_c*tau_m*tau_m*div*Gu[f];
-	}
 }
 
 struct AsmArgs {
@@ -896,89 +807,6 @@ __global__ void FaceMassKernel(int count, int stride, const int* __restrict__ fe
 	}
 }
 
-// Residual-only assembly from the basis table, for elements of at most 32
-// basis functions: one workgroup of 256 threads per element and no slabs.
-// Phase A: four lanes per point sum the fields over the basis functions and
-// the first of them stores the point record; phase B: eight lanes per basis
-// function sum its residual rows over the 64 points in a fixed order, so the
-// result is deterministic.  Without the LDS basis staging and tangent
-// registers of AssembleNsKernel, several elements share a compute unit.
-constexpr int kQr = 35;  // point record r[0..33] in LDS, odd stride
-
-__global__ void __launch_bounds__(kThreads, 2) NsResidualKernel(AsmArgs args)
-{
-	__shared__ double nodal[32*8];
-	__shared__ double qd[kQ*kQr];
-	__shared__ int lconn[32];
-	const int tid = threadIdx.x;
-	const int item = blockIdx.x;
-	if (item >= args.count) return;
-	const int e = args.elements[item];
-	const int b0 = args.eoff[e];
-	const int nen = args.eoff[e + 1] - b0;
-	const double rho = args.rho, mu = args.mu, dt = args.dt;
-	const double nu = mu/rho;
-	for (int a = tid; a < nen; a += kThreads) {
-		const int node = args.conn[b0 + a];
-		lconn[a] = node;
-		for (int f = 0; f < 4; ++f) nodal[8*a + f] = args.state[4*(size_t)node + f];
-		for (int f = 0; f < 3; ++f) nodal[8*a + 4 + f] = args.previous[4*(size_t)node + f];
-	}
-	__syncthreads();
-	const double* tab = args.table + (size_t)b0*kQ*kTableRec;
-	{
-		const int q = tid >> 2, part = tid & 3;
-		double s[22] = {};
-		for (int a = part; a < nen; a += 4) {
-			const double* bb = tab + ((size_t)q*nen + a)*kTableRec;
-			const double N = bb[0], gx = bb[1], gy = bb[2], gz = bb[3], L = bb[4];
-			const double* un = nodal + 8*a;
-#pragma unroll
-			for (int f = 0; f < 4; ++f) {
-				s[f] += un[f]*N;
-				s[4 + 3*f] += un[f]*gx;
-				s[5 + 3*f] += un[f]*gy;
-				s[6 + 3*f] += un[f]*gz;
-			}
-#pragma unroll
-			for (int c = 0; c < 3; ++c) {
-				s[16 + c] += un[c]*L;
-				s[19 + c] += un[4 + c]*N;
-			}
-		}
-#pragma unroll
-		for (int i = 0; i < 22; ++i) {
-			s[i] += __shfl_xor(s[i], 1, 64);
-			s[i] += __shfl_xor(s[i], 2, 64);
-		}
-		if (part == 0)
-			PointRecord<kQ>(s, args.geometry + (size_t)e*kGeomFields*kQ + q, rho, mu, nu, dt, false, qd + q*kQr);
-	}
-	__syncthreads();
-	if (tid < nen*8) {
-		const int a = tid >> 3, sub = tid & 7;
-		double R[4] = {0.0, 0.0, 0.0, 0.0};
-		for (int q = sub; q < kQ; q += 8) {
-			const double* bb = tab + ((size_t)q*nen + a)*kTableRec;
-			const double* r = qd + q*kQr;
-			const double N = bb[0], gx = bb[1], gy = bb[2], gz = bb[3], m = r[0];
-#pragma unroll
-			for (int c = 0; c < 3; ++c) R[c] -= (N*r[6 + c] + gx*r[9 + 3*c] + gy*r[10 + 3*c] + gz*r[11 + 3*c])*m;
-			R[3] -= (N*r[18] - gx*r[19] - gy*r[20] - gz*r[21])*m;
-		}
-#pragma unroll
-		for (int c = 0; c < 4; ++c) {
-			R[c] += __shfl_xor(R[c], 1, 64);
-			R[c] += __shfl_xor(R[c], 2, 64);
-			R[c] += __shfl_xor(R[c], 4, 64);
-		}
-		if (sub == 0) {
-			const size_t node = lconn[a];
-			for (int c = 0; c < 4; ++c) args.negres[4*node + c] += R[c];
-		}
-	}
-}
-
 // Basis records of every (point, function) of one element per workgroup, in
 // the table layout [q][a][kTableRec] the assembly reads slab by slab.
 __global__ void __launch_bounds__(256) BasisTableKernel(const int* __restrict__ eoff, const int* __restrict__ xoff,
@@ -1079,16 +907,22 @@ void AssembleNs(tfi_mesh* m, const double* state, const double* previous, const 
 	double* negative_residual)
 {
 	const bool exact = p.tangent == TFI_TANGENT_EXACT;
-	const bool jac = jacobian != nullptr;
 	const int nen_max = m->max_nen;
 	if (nen_max > kMaxBasis) throw Error("element assembly supports at most 80 basis functions per element");
+	tfi_ctx* ctx = m->ctx;
+	if (!jacobian) {
+		StreamTimer timer(ctx, &ctx->timers.residual_ms);
+		AssembleResidual(m, state, previous, p, negative_residual);
+		ctx->timers.residual_calls += 1;
+		ctx->timers.residual_flops += AssemblyFlops(m, false, exact);
+		return;
+	}
 	const bool table = m->basis_table.size() > 0;
 	// elements of at most 32 basis functions take the FP64-MFMA tangent, which
 	// reads the basis table (evaluating the basis in the same kernel would
 	// push it past its 256 registers)
-	const bool mfma = jac && nen_max <= 32 && table;
-	tfi_ctx* ctx = m->ctx;
-	if (jacobian) Fill(ctx, jacobian, 0.0, m->nnzb*16);
+	const bool mfma = nen_max <= 32 && table;
+	Fill(ctx, jacobian, 0.0, m->nnzb*16);
 	Fill(ctx, negative_residual, 0.0, 4LL*m->nodes);
 	const int tiles_b = (nen_max + 1)/2;
 	int a_tile = mfma ? nen_max : std::min(nen_max, 2*(kThreads/tiles_b));
@@ -1127,33 +961,18 @@ void AssembleNs(tfi_mesh* m, const double* state, const double* previous, const 
 	a.table = table ? m->basis_table.data() : nullptr;
 	a.qstride = qstride;
 	a.max_nen = nen_max;
-	StreamTimer timer(ctx, jac ? &ctx->timers.assembly_ms : &ctx->timers.residual_ms);
-	if (!jac && table && nen_max <= 32) {
-		for (int c = 0; c < m->colors; ++c) {
-			a.elements = m->color_elements.data() + m->color_offsets[c];
-			a.count = m->color_offsets[c + 1] - m->color_offsets[c];
-			if (a.count == 0) continue;
-			hipLaunchKernelGGL(NsResidualKernel, dim3(a.count), dim3(kThreads), 0, ctx->stream, a);
-			TFI_LAUNCH_CHECK("NsResidualKernel");
-		}
-	} else if (mfma) {
+	StreamTimer timer(ctx, &ctx->timers.assembly_ms);
+	if (mfma) {
 		if (exact) LaunchAssembly<true, true, true, 32>(m, a, tiles, lds);
 		else LaunchAssembly<false, true, true, 32>(m, a, tiles, lds);
-	} else if (!jac) {
-		LaunchVectorAssembly<false, false>(m, a, tiles, lds, slab);
 	} else if (exact) {
 		LaunchVectorAssembly<true, true>(m, a, tiles, lds, slab);
 	} else {
 		LaunchVectorAssembly<false, true>(m, a, tiles, lds, slab);
 	}
-	if (jac) {
-		ctx->timers.assembly_calls += 1;
-		ctx->timers.assembly_launches += m->colors;
-		ctx->timers.assembly_flops += AssemblyFlops(m, true, exact);
-	} else {
-		ctx->timers.residual_calls += 1;
-		ctx->timers.residual_flops += AssemblyFlops(m, false, exact);
-	}
+	ctx->timers.assembly_calls += 1;
+	ctx->timers.assembly_launches += m->colors;
+	ctx->timers.assembly_flops += AssemblyFlops(m, true, exact);
 }
 
 // Counted arithmetic of AssembleNsKernel per element with nen basis functions

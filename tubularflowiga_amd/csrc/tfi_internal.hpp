@@ -146,6 +146,10 @@ struct tfi_mesh {
 	std::vector<int> h_color;                // colour per element
 	tfi::DevBuf<long long> pair_offsets;     // [E+1]
 	tfi::DevBuf<int> pair_block;             // [sum nen^2]
+	// per node, the (element, basis function) entries of conn that hold it, ascending
+	tfi::DevBuf<int> node_offsets, node_entries;
+	// residual rows per entry [basis_entries][4], the node sums' input (allocated by the first assembly)
+	tfi::DevBuf<double> element_rows;
 	// geometry [E][kGeomFields][64]
 	tfi::DevBuf<double> geometry;
 	// optional precomputed basis records: element e at eoff[e]*64*5, [q][a][5]
@@ -217,6 +221,9 @@ struct NsParams {
 	int tangent = TFI_TANGENT_LEGACY;
 };
 void AssembleNs(tfi_mesh* mesh, const double* state, const double* previous, const NsParams& p, double* jacobian,
+	double* negative_residual);
+// The negated residual alone (tfi_residual.hip).
+void AssembleResidual(tfi_mesh* mesh, const double* state, const double* previous, const NsParams& p,
 	double* negative_residual);
 double AssemblyFlops(const tfi_mesh* mesh, bool with_jacobian, bool exact);
 // Builds (enable) or frees the per-element basis table; enable < 0 builds it

@@ -230,10 +230,18 @@ void BuildMesh(tfi_mesh* m)
 	for (int n = 0; n < N; ++n) n2e_off[n + 1] += n2e_off[n];
 	std::vector<int> n2e(n2e_off[N]);
 	{
-		std::vector<int> fill(n2e_off.begin(), n2e_off.end() - 1);
+		std::vector<int> fill(n2e_off.begin(), n2e_off.end() - 1), entries(n2e_off[N]);
 		for (int e = 0; e < E; ++e)
-			for (int a = m->h_eoff[e]; a < m->h_eoff[e + 1]; ++a) n2e[fill[m->h_conn[a]]++] = e;
+			for (int a = m->h_eoff[e]; a < m->h_eoff[e + 1]; ++a) {
+				const int at = fill[m->h_conn[a]]++;
+				n2e[at] = e;
+				entries[at] = a;
+			}
+		m->node_entries.Allocate(ctx, entries.size());
+		m->node_entries.Upload(entries.data(), entries.size());
 	}
+	m->node_offsets.Allocate(ctx, N + 1);
+	m->node_offsets.Upload(n2e_off.data(), N + 1);
 	int max_candidates = 0;
 	for (int n = 0; n < N; ++n) {
 		int c = 0;
@@ -242,12 +250,11 @@ void BuildMesh(tfi_mesh* m)
 	}
 	const int capacity = NextPow2(std::max(max_candidates, 2));
 	if (capacity > 16384) throw Error("node couples too many element bases for the LDS pattern builder");
-	DevBuf<int> d_n2e_off(ctx, N + 1), d_n2e(ctx, n2e.size()), row_len(ctx, N), status(ctx, 1);
-	d_n2e_off.Upload(n2e_off.data(), N + 1);
+	DevBuf<int> d_n2e(ctx, n2e.size()), row_len(ctx, N), status(ctx, 1);
 	d_n2e.Upload(n2e.data(), n2e.size());
 	FillInt(ctx, status.data(), 0, 1);
 	const size_t lds = capacity*sizeof(int);
-	hipLaunchKernelGGL(PatternKernel, dim3(N), dim3(256), lds, ctx->stream, N, d_n2e_off.data(), d_n2e.data(),
+	hipLaunchKernelGGL(PatternKernel, dim3(N), dim3(256), lds, ctx->stream, N, m->node_offsets.data(), d_n2e.data(),
 		m->eoff.data(), m->conn.data(), capacity, 0, row_len.data(), nullptr, nullptr, nullptr, status.data());
 	TFI_LAUNCH_CHECK("PatternKernel count");
 	int st = 0;
@@ -267,7 +274,7 @@ void BuildMesh(tfi_mesh* m)
 	m->row_offsets.Upload(ro.data(), N + 1);
 	m->columns.Allocate(ctx, total);
 	m->diagonal.Allocate(ctx, N);
-	hipLaunchKernelGGL(PatternKernel, dim3(N), dim3(256), lds, ctx->stream, N, d_n2e_off.data(), d_n2e.data(),
+	hipLaunchKernelGGL(PatternKernel, dim3(N), dim3(256), lds, ctx->stream, N, m->node_offsets.data(), d_n2e.data(),
 		m->eoff.data(), m->conn.data(), capacity, 1, nullptr, m->row_offsets.data(), m->columns.data(),
 		m->diagonal.data(), status.data());
 	TFI_LAUNCH_CHECK("PatternKernel fill");
