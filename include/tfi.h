@@ -442,8 +442,8 @@ int tfi_solve_bench_spmv(tfi_solve* solve, int repetitions, double* milliseconds
 typedef struct {
 	double spmv_ms, spmv_calls, spmv_bytes;           /* fine-level fp64 SpMV */
 	double spmv32_ms, spmv32_calls, spmv32_bytes;     /* fine-level fp32 SpMV */
-	double assembly_ms, assembly_calls, assembly_flops;  /* residual + tangent: AssembleNsKernel launches */
-	double assembly_launches;                         /* (one launch per element colour) */
+	double assembly_ms, assembly_calls, assembly_flops;  /* residual + tangent */
+	double assembly_launches;                         /* tangent launches: one, or one per element colour on large meshes */
 	double residual_ms, residual_calls, residual_flops;  /* residual-only assemblies */
 	double spmv2_ms, spmv2_calls, spmv2_bytes;        /* transport 2x2 fp64 SpMV */
 	double transport_assembly_ms;                     /* transport L and P assembly (all colours) */

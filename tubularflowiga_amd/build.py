@@ -26,7 +26,7 @@ LIB = PKG / "libtfi_hip.so"
 CLI = PKG / "iga_hip"
 PACK = PKG / "tfi_pack"
 
-SOURCES = ["tfi_core.hip", "tfi_mesh.hip", "tfi_assembly.hip", "tfi_residual.hip", "tfi_sparse.hip", "tfi_krylov.hip",
+SOURCES = ["tfi_core.hip", "tfi_mesh.hip", "tfi_assembly.hip", "tfi_residual.hip", "tfi_tangent.hip", "tfi_sparse.hip", "tfi_krylov.hip",
            "tfi_amg.hip", "tfi_mlp.hip", "tfi_warmstart.hip", "tfi_flow.hip", "tfi_transport.hip",
            "tfi_solve.hip"]
 

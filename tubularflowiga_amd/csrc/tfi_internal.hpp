@@ -150,6 +150,12 @@ struct tfi_mesh {
 	tfi::DevBuf<int> node_offsets, node_entries;
 	// residual rows per entry [basis_entries][4], the node sums' input (allocated by the first assembly)
 	tfi::DevBuf<double> element_rows;
+	// tangent assembly of meshes whose staged element blocks fit: the blocks [element_pairs][16] and, per
+	// pattern block, its (element, a, b) pairs, ascending (allocated by the first tangent assembly)
+	int staged = -1;                         // -1: not decided yet
+	tfi::DevBuf<double> staging;
+	tfi::DevBuf<int> block_offsets, block_pairs;
+	tfi::DevBuf<double> point_records;       // of one tangent launch
 	// geometry [E][kGeomFields][64]
 	tfi::DevBuf<double> geometry;
 	// optional precomputed basis records: element e at eoff[e]*64*5, [q][a][5]
@@ -222,9 +228,13 @@ struct NsParams {
 };
 void AssembleNs(tfi_mesh* mesh, const double* state, const double* previous, const NsParams& p, double* jacobian,
 	double* negative_residual);
-// The negated residual alone (tfi_residual.hip).
-void AssembleResidual(tfi_mesh* mesh, const double* state, const double* previous, const NsParams& p,
-	double* negative_residual);
+// Negated residual rows of `count` elements (ids in `elements`, or the first
+// `count` elements when null) into mesh->element_rows and, unless null, the
+// point records of the tangent into points (tfi_residual.hip); then the node
+// sums of all elements' rows.
+void ElementResiduals(tfi_mesh* mesh, const double* state, const double* previous, const NsParams& p,
+	const int* elements, int count, double* points);
+void SumResiduals(tfi_mesh* mesh, double* negative_residual);
 double AssemblyFlops(const tfi_mesh* mesh, bool with_jacobian, bool exact);
 // Builds (enable) or frees the per-element basis table; enable < 0 builds it
 // when it takes at most half of the free device memory.

@@ -18,15 +18,60 @@ __device__ inline void Bern3(double x, double b[4], double db[4], double d2b[4])
 	d2b[0] = 6.0*y; d2b[1] = -12.0 + 18.0*x; d2b[2] = 6.0 - 18.0*x; d2b[3] = 6.0*x;
 }
 
+constexpr int kTableRec = 5;  // N, dN/dx, dN/dy, dN/dz, lap N
+
+// What the tangent needs of a point, written by the residual kernel as
+// [item][kTangentRec][kQ]: measure, tau_M, tau_C, u, u', grad u, G u.
+constexpr int kTangentRec = 21;
+
+// Value, physical gradient and Laplacian of the basis function with Bezier
+// extraction row c[64] at element point q (Bernstein sum-factorisation in
+// xi, eta, zeta; gq = geometry record of the point, field stride kQ).
+__device__ inline void EvalBasis(const double* __restrict__ c, const double* __restrict__ gq, int q,
+	double out[kTableRec])
+{
+	double bx[4], dbx[4], d2bx[4], by[4], dby[4], d2by[4], bz[4], dbz[4], d2bz[4];
+	Bern3(kGp[q & 3], bx, dbx, d2bx);
+	Bern3(kGp[(q >> 2) & 3], by, dby, d2by);
+	Bern3(kGp[q >> 4], bz, dbz, d2bz);
+	double v = 0, g0 = 0, g1 = 0, g2 = 0, h00 = 0, h11 = 0, h22 = 0, h01 = 0, h02 = 0, h12 = 0;
+	for (int k = 0; k < 4; ++k) {
+		double s00 = 0, s10 = 0, s01 = 0, s20 = 0, s11 = 0, s02 = 0;
+		for (int j = 0; j < 4; ++j) {
+			const double* cr = c + 16*k + 4*j;
+			const double x0 = cr[0]*bx[0] + cr[1]*bx[1] + cr[2]*bx[2] + cr[3]*bx[3];
+			const double x1 = cr[0]*dbx[0] + cr[1]*dbx[1] + cr[2]*dbx[2] + cr[3]*dbx[3];
+			const double x2 = cr[0]*d2bx[0] + cr[1]*d2bx[1] + cr[2]*d2bx[2] + cr[3]*d2bx[3];
+			s00 += x0*by[j]; s10 += x1*by[j]; s20 += x2*by[j];
+			s01 += x0*dby[j]; s11 += x1*dby[j]; s02 += x0*d2by[j];
+		}
+		v += s00*bz[k]; g0 += s10*bz[k]; g1 += s01*bz[k]; g2 += s00*dbz[k];
+		h00 += s20*bz[k]; h11 += s02*bz[k]; h22 += s00*d2bz[k];
+		h01 += s11*bz[k]; h02 += s10*dbz[k]; h12 += s01*dbz[k];
+	}
+	double inv[9];
+#pragma unroll
+	for (int i = 0; i < 9; ++i) inv[i] = gq[(1 + i)*kQ];
+	out[0] = v;
+	out[1] = g0*inv[0] + g1*inv[3] + g2*inv[6];
+	out[2] = g0*inv[1] + g1*inv[4] + g2*inv[7];
+	out[3] = g0*inv[2] + g1*inv[5] + g2*inv[8];
+	out[4] = h00*gq[10*kQ] + h11*gq[11*kQ] + h22*gq[12*kQ]
+		+ 2.0*(h01*gq[13*kQ] + h02*gq[14*kQ] + h12*gq[15*kQ])
+		+ g0*gq[16*kQ] + g1*gq[17*kQ] + g2*gq[18*kQ];
+}
+
 // Per-point record from the field sums s (u, p, grad u, grad p, lap u, u_prev
 // at the point; 22 values) and the point's geometry record gq (fields 0..9:
-// measure and J^-1, field stride kGs): r[0] measure, r[1..2] tau_M, tau_C, r[3..5] u, r[6..8] rho (du/dt +
-// w.grad u), r[9..17] stress rows, r[18] div u, r[19..21] u', r[22..24] w =
-// u + u', r[25..33] grad u and, with exact_tangent, r[34..54] the
-// linearisation of u' (K, R, c1) the consistent tangent needs.
+// measure and J^-1, field stride kGs): r[0] measure, r[1..2] tau_M, tau_C,
+// r[3..5] u, r[6..8] rho (du/dt + w.grad u), r[9..17] stress rows, r[18] div u,
+// r[19..21] u', r[22..24] w = u + u', r[25..33] grad u, r[34..36] G u with
+// G = J^-T J^-1.
+constexpr int kPointRecord = 37;
+
 template <int kGs>
 __device__ inline void PointRecord(const double* __restrict__ s, const double* __restrict__ gq, double rho, double mu,
-	double nu, double dt, bool exact_tangent, double* __restrict__ r)
+	double nu, double dt, double* __restrict__ r)
 {
 	double inv[3][3];
 	for (int a = 0; a < 3; ++a)
@@ -77,25 +122,7 @@ __device__ inline void PointRecord(const double* __restrict__ s, const double* _
 	for (int c = 0; c < 3; ++c) r[22 + c] = w[c];
 	for (int c = 0; c < 3; ++c)
 		for (int d = 0; d < 3; ++d) r[25 + 3*c + d] = grad[c][d];
-	if (exact_tangent) {
-		// d(u')/d(u_f) = N_b K[.][f] - delta tau_M s_b with
-		// K_cf = tau_M^3 strong_c (G u)_f - tau_M du_c/dx_f, and
-		// R = grad u + grad u K, c1_f = rho tau_C tau_M^2 div (G u)_f.
-		double Gu[3];
-		for (int i = 0; i < 3; ++i) Gu[i] = G[i][0]*u[0] + G[i][1]*u[1] + G[i][2]*u[2];
-		const double tm3 = tau_m*tau_m*tau_m;
-		double K[3][3];
-		for (int c = 0; c < 3; ++c) {
-			const double strong = -fu[c]/tau_m;
-			for (int f = 0; f < 3; ++f) K[c][f] = tm3*strong*Gu[f] - tau_m*grad[c][f];
-		}
-		for (int c = 0; c < 3; ++c)
-			for (int f = 0; f < 3; ++f) {
-				r[34 + 3*c + f] = K[c][f];
-				r[43 + 3*c + f] = grad[c][f] + grad[c][0]*K[0][f] + grad[c][1]*K[1][f] + grad[c][2]*K[2][f];
-			}
-		for (int f = 0; f < 3; ++f) r[52 + f] = rho*tau_c*tau_m*tau_m*div*Gu[f];
-	}
+	for (int i = 0; i < 3; ++i) r[34 + i] = G[i][0]*u[0] + G[i][1]*u[1] + G[i][2]*u[2];
 }
 
 }  // namespace

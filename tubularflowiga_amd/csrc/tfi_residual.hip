@@ -34,7 +34,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kFields = 22;  // u (3), p, grad u (9), grad p (3), lap u (3), u_prev (3): the order PointRecord takes
-constexpr int kQr = 34;      // entries of the point record the residual uses
 
 struct ResidualArgs {
 	const int* eoff;
@@ -46,7 +45,9 @@ struct ResidualArgs {
 	const double* state;
 	const double* previous;
 	double rho, mu, dt;
-	double* rows;  // [entries][4]
+	double* rows;         // [entries][4]
+	const int* elements;  // element ids of this launch, or null: all in order
+	double* points;       // tangent records [workgroup][kTangentRec][kQ], or null
 };
 
 // LDS in doubles: P holds, in turn, the dense extraction rows [nen][64], the
@@ -66,7 +67,7 @@ __global__ void __launch_bounds__(kThreads) NsResidualKernel(ResidualArgs args, 
 	double* nodal = Q + kQDoubles;       // [nen][u, u_prev, v, v_prev, w, w_prev, p, 0]
 	double* tab = nodal + 8*max_nen;     // [B, B', B''][Gauss point][Bernstein index]
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int e = blockIdx.x;
+	const int e = args.elements ? args.elements[blockIdx.x] : blockIdx.x;
 	const int b0 = args.eoff[e];
 	const int nen = args.eoff[e + 1] - b0;
 	for (int i = tid; i < nen*64; i += kThreads) P[i] = 0.0;
@@ -193,10 +194,22 @@ __global__ void __launch_bounds__(kThreads) NsResidualKernel(ResidualArgs args, 
 	// fluxes at the points: the factor of N_a and, pulled back to the parametric
 	// directions, that of grad N_a, times the measure
 	if (wave == 0) {
-		double s[kFields], r[kQr];
+		double s[kFields], r[kPointRecord];
 #pragma unroll
 		for (int i = 0; i < kFields; ++i) s[i] = Q[i*64 + lane];
-		PointRecord<kQ>(s, gq, args.rho, args.mu, args.mu/args.rho, args.dt, false, r);
+		PointRecord<kQ>(s, gq, args.rho, args.mu, args.mu/args.rho, args.dt, r);
+		if (args.points) {
+			double* o = args.points + (size_t)blockIdx.x*kTangentRec*kQ + lane;
+#pragma unroll
+			for (int i = 0; i < 6; ++i) o[i*kQ] = r[i];
+#pragma unroll
+			for (int i = 0; i < 3; ++i) {
+				o[(6 + i)*kQ] = r[19 + i];
+				o[(18 + i)*kQ] = r[34 + i];
+			}
+#pragma unroll
+			for (int i = 0; i < 9; ++i) o[(9 + i)*kQ] = r[25 + i];
+		}
 		double inv[3][3];
 #pragma unroll
 		for (int i = 0; i < 9; ++i) inv[i/3][i%3] = gq[(1 + i)*kQ];
@@ -275,21 +288,27 @@ __global__ void __launch_bounds__(kThreads) NodeSumKernel(int nodes, const int* 
 
 }  // namespace
 
-void AssembleResidual(tfi_mesh* m, const double* state, const double* previous, const NsParams& p,
-	double* negative_residual)
+void ElementResiduals(tfi_mesh* m, const double* state, const double* previous, const NsParams& p, const int* elements,
+	int count, double* points)
 {
+	if (count == 0) return;
 	tfi_ctx* ctx = m->ctx;
 	if (!m->element_rows.size()) m->element_rows.Allocate(ctx, 4*(size_t)m->basis_entries);
 	ResidualArgs a{m->eoff.data(), m->conn.data(), m->xoff.data(), m->xcol.data(), m->xval.data(), m->geometry.data(),
-		state, previous, p.density, p.viscosity, p.dt, m->element_rows.data()};
+		state, previous, p.density, p.viscosity, p.dt, m->element_rows.data(), elements, points};
 	const int nen = m->max_nen;
 	const size_t lds = sizeof(double)*(PDoubles(nen) + kQDoubles + 8*(size_t)nen + 48);
 	static_assert(sizeof(double)*(PDoubles(kMaxBasis) + kQDoubles + 8*kMaxBasis + 48) <= 65536,
 		"the largest element fits the default dynamic LDS");
-	hipLaunchKernelGGL(NsResidualKernel, dim3(m->elements), dim3(kThreads), lds, ctx->stream, a, nen);
+	hipLaunchKernelGGL(NsResidualKernel, dim3(count), dim3(kThreads), lds, ctx->stream, a, nen);
 	TFI_LAUNCH_CHECK("NsResidualKernel");
-	hipLaunchKernelGGL(NodeSumKernel, dim3((4LL*m->nodes + kThreads - 1)/kThreads), dim3(kThreads), 0, ctx->stream,
-		m->nodes, m->node_offsets.data(), m->node_entries.data(), m->element_rows.data(), negative_residual);
+}
+
+void SumResiduals(tfi_mesh* m, double* negative_residual)
+{
+	hipLaunchKernelGGL(NodeSumKernel, dim3(static_cast<unsigned>((4LL*m->nodes + kThreads - 1)/kThreads)),
+		dim3(kThreads), 0, m->ctx->stream, m->nodes, m->node_offsets.data(), m->node_entries.data(),
+		m->element_rows.data(), negative_residual);
 	TFI_LAUNCH_CHECK("NodeSumKernel");
 }
 
