@@ -371,86 +371,169 @@ __global__ void GalerkinKernel(long long cblocks, const long long* __restrict__ 
 	coarse[(size_t)K*16 + e] = s;
 }
 
-// Augmented [A | I] of the coarsest level (n = 4 rows, leading dimension 2n),
-// on a zero-filled buffer: aug[(4i+a)*2n + 4j+b] = A_ij[a][b], identity on the right.
-__global__ void DenseAugKernel(int rows, const int* __restrict__ ro, const int* __restrict__ cols,
-	const double* __restrict__ vals, double* __restrict__ aug)
+// The coarsest level as a dense matrix, on a zero-filled n x n buffer (n = 4 rows).
+__global__ void DenseKernel(int rows, const int* __restrict__ ro, const int* __restrict__ cols,
+	const double* __restrict__ vals, double* __restrict__ dense)
 {
 	const int i = blockIdx.x;
-	const int n = 4*rows, w = 2*n;
+	const int n = 4*rows;
 	for (int k = ro[i]; k < ro[i + 1]; ++k)
-		for (int e = threadIdx.x; e < 16; e += blockDim.x) {
-			const int a = e >> 2, b = e & 3;
-			aug[(size_t)(4*i + a)*w + 4*cols[k] + b] = vals[(size_t)k*16 + e];
-		}
-	if (threadIdx.x < 4) aug[(size_t)(4*i + threadIdx.x)*w + n + 4*i + threadIdx.x] = 1.0;
+		for (int e = threadIdx.x; e < 16; e += blockDim.x)
+			dense[(size_t)(4*i + (e >> 2))*n + 4*cols[k] + (e & 3)] = vals[(size_t)k*16 + e];
 }
 
-// Gauss-Jordan step p, part 1 (one workgroup): partial pivot search in column
-// p over rows >= p (largest magnitude, lowest row on ties), row swap, scaling
-// of the pivot row, and the elimination multipliers m[i] = aug[i][p] (i != p).
-__global__ void __launch_bounds__(1024) PivotKernel(int n, int p, double* __restrict__ aug, double* __restrict__ mult,
+// Dense inverse by in-place Gauss-Jordan elimination with partial pivoting, in
+// panels of kPanel columns: no row is moved, column p is exchanged with the row
+// r_p it is pivoted on, and at the end inverse[p][r_k] = matrix[r_p][k].
+//
+// Bound by latency: a pivot needs the column of the pivot before.  A launch
+// per pivot plus one for the elimination cost 10.7 us each pivot (676 rows: 7.3
+// ms); a panel keeps its columns in the registers of one workgroup, a row per
+// thread, where a pivot is one barrier (20.8 us for 16 pivots and the launch),
+// and the columns outside the panel take all its pivots as one product of rank
+// kPanel over the whole grid (7.3 us): 1.2 ms.  16 columns: 32 registers of a
+// thread's 128 at 1024 threads.
+constexpr int kPanel = 16;
+constexpr int kDenseMax = 1024;   // rows the panel's workgroup holds
+constexpr int kUpdateRows = 32;   // rows of a workgroup of PanelUpdateKernel
+
+// Largest value over the wave (0 where a lane has no source), the same in every lane.
+__device__ inline unsigned int WaveMax(unsigned int v)
+{
+	v = max(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));  // row_shr:1
+	v = max(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));  // row_shr:2
+	v = max(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));  // row_shr:4
+	v = max(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));  // row_shr:8
+	v = max(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+	v = max(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+	return (unsigned int)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Pivots columns p0 .. p0 + width - 1.  step[i] is the column row i is pivot
+// of, n if none yet; pivot[p] the pivot row of column p; w[t][i] the panel's
+// columns afterwards, column by column.  The pivot is the row of the largest
+// magnitude to 20 bits of the significand (the upper word of the entry orders
+// them), the lowest row on ties.  Every wave offers its best row, scaled as
+// pivot row, and after one barrier all threads choose among the at most 16
+// offers.  A thread's row is rotated by one column per pivot, so that the loop
+// indexes registers by constants and stays small: unrolled over the panel's 16
+// pivots the code (35 KB) ran at the rate it was fetched.  The panel is read and
+// written by columns (in[row*row_stride + t*column_stride]): neighbouring
+// threads, neighbouring addresses.
+__global__ void __launch_bounds__(kDenseMax) PanelKernel(int n, int p0, int width, const double* __restrict__ in,
+	int row_stride, int column_stride, double* __restrict__ w, int* __restrict__ step, int* __restrict__ pivot,
 	int* __restrict__ status)
 {
-	__shared__ double sval[1024];
-	__shared__ int sidx[1024];
-	const int w = 2*n;
-	double best = -1.0;
-	int bi = p;
-	for (int i = p + threadIdx.x; i < n; i += blockDim.x) {
-		const double v = fabs(aug[(size_t)i*w + p]);
-		if (v > best) { best = v; bi = i; }
-	}
-	sval[threadIdx.x] = best;
-	sidx[threadIdx.x] = bi;
+	constexpr int kWaves = kDenseMax/64;
+	__shared__ unsigned int key[2][kWaves];
+	__shared__ int key_row[2][kWaves];
+	__shared__ double offer[2][kWaves][kPanel];
+	const int i = threadIdx.x, lane = i & 63, wave = i >> 6;
+	if (i < 2*kWaves) key[i/kWaves][i % kWaves] = 0;  // waves the workgroup does not have
+	int mine = i < n ? step[i] : 0;
+	double a[kPanel];
+#pragma unroll
+	for (int t = 0; t < kPanel; ++t)
+		a[t] = i < n && t < width ? in[(size_t)i*row_stride + (size_t)t*column_stride] : 0.0;
 	__syncthreads();
-	for (int s = blockDim.x/2; s > 0; s >>= 1) {
-		if (threadIdx.x < s) {
-			const double o = sval[threadIdx.x + s];
-			const int oi = sidx[threadIdx.x + s];
-			if (o > sval[threadIdx.x] || (o == sval[threadIdx.x] && oi < sidx[threadIdx.x])) {
-				sval[threadIdx.x] = o;
-				sidx[threadIdx.x] = oi;
-			}
+#pragma unroll 1
+	for (int c = 0; c < width; ++c) {
+		const int buf = c & 1;
+		// a row without a pivot: 1 + upper word of |entry| (1 for a NaN, which is never chosen over a number)
+		unsigned int k = 0;
+		if (mine == n) k = a[0] == a[0] ? 1u + ((unsigned int)__double2hiint(a[0]) & 0x7fffffffu) : 1u;
+		const double inv = a[0] != 0.0 ? 1.0/a[0] : 0.0;
+		const unsigned int m = WaveMax(k);
+		const int first = __ffsll(__ballot(k == m)) - 1;
+		if (lane == first) {
+			key[buf][wave] = m;
+			key_row[buf][wave] = i;
+			offer[buf][wave][0] = inv;
+#pragma unroll
+			for (int t = 1; t < kPanel; ++t) offer[buf][wave][t] = a[t]*inv;
 		}
 		__syncthreads();
-	}
-	const int q = sidx[0];
-	if (threadIdx.x == 0 && (!(sval[0] > 1e-300) || !isfinite(sval[0]))) *status = 1;
-	if (q != p)
-		for (int j = threadIdx.x; j < w; j += blockDim.x) {
-			const double t = aug[(size_t)p*w + j];
-			aug[(size_t)p*w + j] = aug[(size_t)q*w + j];
-			aug[(size_t)q*w + j] = t;
+		// lane l of every wave reads offer l; the pivot row goes through scalar registers
+		const unsigned int o = key[buf][lane & (kWaves - 1)];
+		const int win = __ffsll(__ballot(o == WaveMax(o))) - 1;
+		const int chosen = __builtin_amdgcn_readlane(key_row[buf][lane & (kWaves - 1)], win);
+		const double part = offer[buf][win][lane & (kPanel - 1)];
+		double row[kPanel];
+#pragma unroll
+		for (int t = 0; t < kPanel; ++t)
+			row[t] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(part), t),
+				__builtin_amdgcn_readlane(__double2loint(part), t));
+		const double f = a[0];
+		if (i == chosen) {
+			if (!(fabs(f) > 1e-300) || !isfinite(f)) *status = 1;
+			mine = p0 + c;
+			pivot[p0 + c] = i;
+#pragma unroll
+			for (int t = 1; t < kPanel; ++t) a[t - 1] = row[t];
+			a[kPanel - 1] = row[0];
+		} else {
+#pragma unroll
+			for (int t = 1; t < kPanel; ++t) a[t - 1] = a[t] - f*row[t];
+			a[kPanel - 1] = -f*row[0];
 		}
-	__syncthreads();
-	const double piv = aug[(size_t)p*w + p];
-	const double inv = piv != 0.0 ? 1.0/piv : 0.0;
-	__syncthreads();
-	for (int j = threadIdx.x; j < w; j += blockDim.x) aug[(size_t)p*w + j] *= inv;
-	for (int i = threadIdx.x; i < n; i += blockDim.x) mult[i] = i == p ? 0.0 : aug[(size_t)i*w + p];
+	}
+	if (i < n) {
+		step[i] = mine;
+#pragma unroll
+		for (int t = 0; t < kPanel; ++t) w[(size_t)((t + width) % kPanel)*n + i] = a[t];
+	}
 }
 
-// Gauss-Jordan step p, part 2 (whole grid): aug[i][j] -= m[i] aug[p][j] for
-// i != p; column p of the other rows becomes exactly zero.
-__global__ void EliminateKernel(int n, int p, double* __restrict__ aug, const double* __restrict__ mult)
+// The panel's pivots applied to the whole matrix, from one buffer to another:
+// out[i][j] = (row i is a pivot of the panel ? 0 : in[i][j]) + sum_t w[t][i] in[pivot[p0 + t]][j],
+// and the panel's own columns are w.  The columns of the next panel go to next
+// as well, column by column.
+__global__ void __launch_bounds__(256) PanelUpdateKernel(int n, int p0, int width, const double* __restrict__ in,
+	const double* __restrict__ w, const int* __restrict__ step, const int* __restrict__ pivot, double* __restrict__ out,
+	double* __restrict__ next)
 {
-	const int w = 2*n;
-	const long long t = blockIdx.x*(long long)blockDim.x + threadIdx.x;
-	if (t >= (long long)n*w) return;
-	const int i = static_cast<int>(t/w), j = static_cast<int>(t - (long long)i*w);
-	if (i == p) return;
-	aug[t] = j == p ? 0.0 : aug[t] - mult[i]*aug[(size_t)p*w + j];
+	constexpr int kRows = kUpdateRows/4;  // rows of a wave
+	__shared__ double ws[kUpdateRows][kPanel + 1];
+	__shared__ int keep[kUpdateRows];
+	__shared__ double ps[kPanel][64];  // the pivot rows
+	const int j = blockIdx.x*64 + (threadIdx.x & 63), i0 = blockIdx.y*kUpdateRows;
+	for (int k = threadIdx.x; k < kUpdateRows*kPanel; k += 256)
+		ws[k % kUpdateRows][k/kUpdateRows] = i0 + k % kUpdateRows < n ? w[(size_t)(k/kUpdateRows)*n + i0 + k % kUpdateRows] : 0.0;
+	if (threadIdx.x < kUpdateRows) {
+		const int s = i0 + threadIdx.x < n ? step[i0 + threadIdx.x] : 0;
+		keep[threadIdx.x] = !(s >= p0 && s < p0 + width);
+	}
+	for (int t = threadIdx.x >> 6; t < kPanel; t += 4)
+		ps[t][threadIdx.x & 63] = t < width && j < n ? in[(size_t)pivot[p0 + t]*n + j] : 0.0;
+	__syncthreads();
+	if (j >= n) return;
+	const int r0 = (threadIdx.x >> 6)*kRows;
+	const bool panel = j >= p0 && j < p0 + width;
+	double acc[kRows];
+#pragma unroll
+	for (int r = 0; r < kRows; ++r) acc[r] = i0 + r0 + r < n && keep[r0 + r] ? in[(size_t)(i0 + r0 + r)*n + j] : 0.0;
+#pragma unroll 4
+	for (int t = 0; t < kPanel; ++t) {
+		const double p = ps[t][threadIdx.x & 63];
+#pragma unroll
+		for (int r = 0; r < kRows; ++r) acc[r] += ws[r0 + r][t]*p;
+	}
+#pragma unroll
+	for (int r = 0; r < kRows; ++r)
+		if (i0 + r0 + r < n) {
+			out[(size_t)(i0 + r0 + r)*n + j] = panel ? ws[r0 + r][j - p0] : acc[r];
+			if (j >= p0 + kPanel && j < p0 + 2*kPanel) next[(size_t)(j - p0 - kPanel)*n + i0 + r0 + r] = acc[r];
+		}
 }
 
-// inverse (n x n) from the right half of the augmented matrix, in T
+// inverse (n x n, in T) from the eliminated matrix: inverse[p][r_k] = matrix[r_p][k], one row p per workgroup
 template <class T>
-__global__ void ExtractInverseKernel(int n, const double* __restrict__ aug, T* __restrict__ inv)
+__global__ void ExtractInverseKernel(int n, const double* __restrict__ matrix, const int* __restrict__ pivot,
+	T* __restrict__ inv)
 {
-	const long long t = blockIdx.x*(long long)blockDim.x + threadIdx.x;
-	if (t >= (long long)n*n) return;
-	const int i = static_cast<int>(t/n), j = static_cast<int>(t - (long long)i*n);
-	inv[t] = static_cast<T>(aug[(size_t)i*2*n + n + j]);
+	const int p = blockIdx.x;
+	const double* row = matrix + (size_t)pivot[p]*n;
+	for (int k = threadIdx.x; k < n; k += blockDim.x) inv[(size_t)p*n + pivot[k]] = static_cast<T>(row[k]);
 }
 
 // y = Dinv b (dense), one wave per row
@@ -533,9 +616,9 @@ struct Amg::Impl {
 	bool built = false;
 	std::vector<std::unique_ptr<Level>> L;
 	int nc = 0;  // coarsest dense size (4 * rows)
-	DevBuf<double> aug, mult, dinv64, v64tmp;
+	DevBuf<double> dense[2], panel, next_panel, dinv64;  // the coarsest matrix under elimination, from one buffer to the other
 	DevBuf<float> dinv32;
-	DevBuf<int> status;
+	DevBuf<int> status, pivot, step;
 	DevBuf<int> scale_flags;  // per level: S did not fit FP16
 
 	void Symbolic(const double* fine_values);
@@ -795,9 +878,12 @@ void Amg::Impl::Symbolic(const double* fine_values)
 		}
 	}
 	nc = 4*L.back()->rows;
-	if (nc > 1024) throw Error("AMG coarsest level too large for the dense solve");
-	aug.Allocate(ctx, (size_t)nc*2*nc);
-	mult.Allocate(ctx, nc);
+	if (nc > kDenseMax) throw Error("AMG coarsest level too large for the dense solve");
+	for (auto& d : dense) d.Allocate(ctx, (size_t)nc*nc);
+	panel.Allocate(ctx, (size_t)nc*kPanel);
+	next_panel.Allocate(ctx, (size_t)nc*kPanel);
+	pivot.Allocate(ctx, nc);
+	step.Allocate(ctx, nc);
 	if (precision == TFI_MIXED) dinv32.Allocate(ctx, (size_t)nc*nc);
 	else dinv64.Allocate(ctx, (size_t)nc*nc);
 	status.Allocate(ctx, 1);
@@ -869,30 +955,33 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 		}
 	// coarsest dense inverse, built and inverted on the device
 	Level& c = *L.back();
-	Fill(ctx, aug.data(), 0.0, (long long)nc*2*nc);
-	hipLaunchKernelGGL(DenseAugKernel, dim3(c.rows), dim3(64), 0, ctx->stream, c.rows, c.ro, c.cols, c.vals64,
-		aug.data());
-	TFI_LAUNCH_CHECK("DenseAugKernel");
+	Fill(ctx, dense[0].data(), 0.0, (long long)nc*nc);
+	hipLaunchKernelGGL(DenseKernel, dim3(c.rows), dim3(64), 0, ctx->stream, c.rows, c.ro, c.cols, c.vals64,
+		dense[0].data());
+	TFI_LAUNCH_CHECK("DenseKernel");
 	FillInt(ctx, status.data(), 0, 1);
-	// n pivot steps, each a pivot/scale launch and a grid-wide elimination
-	// launch (the single-workgroup form is bound by one CU's L2 bandwidth)
-	const long long cells = (long long)nc*2*nc;
-	for (int p = 0; p < nc; ++p) {
-		hipLaunchKernelGGL(PivotKernel, dim3(1), dim3(1024), 0, ctx->stream, nc, p, aug.data(), mult.data(),
+	FillInt(ctx, step.data(), nc, nc);
+	const double* matrix = dense[0].data();
+	for (int p0 = 0, flip = 1; p0 < nc; p0 += kPanel, flip ^= 1) {
+		const int width = std::min(kPanel, nc - p0);
+		hipLaunchKernelGGL(PanelKernel, dim3(1), dim3((nc + 63)/64*64), 0, ctx->stream, nc, p0, width,
+			p0 ? next_panel.data() : matrix, p0 ? 1 : nc, p0 ? nc : 1, panel.data(), step.data(), pivot.data(),
 			status.data());
-		hipLaunchKernelGGL(EliminateKernel, dim3(Grid(cells)), dim3(256), 0, ctx->stream, nc, p, aug.data(),
-			mult.data());
+		hipLaunchKernelGGL(PanelUpdateKernel, dim3((nc + 63)/64, (nc + kUpdateRows - 1)/kUpdateRows), dim3(256), 0,
+			ctx->stream, nc, p0, width, matrix, panel.data(), step.data(), pivot.data(), dense[flip].data(),
+			next_panel.data());
+		matrix = dense[flip].data();
 	}
-	TFI_LAUNCH_CHECK("EliminateKernel");
+	TFI_LAUNCH_CHECK("PanelUpdateKernel");
 	int st = 0;
 	status.Download(&st, 1);
 	if (st) throw Error("AMG coarsest operator is singular");
 	if (precision == TFI_MIXED) {
-		hipLaunchKernelGGL(ExtractInverseKernel<float>, dim3(Grid((long long)nc*nc)), dim3(256), 0, ctx->stream, nc,
-			aug.data(), dinv32.data());
+		hipLaunchKernelGGL(ExtractInverseKernel<float>, dim3(nc), dim3(256), 0, ctx->stream, nc, matrix, pivot.data(),
+			dinv32.data());
 	} else {
-		hipLaunchKernelGGL(ExtractInverseKernel<double>, dim3(Grid((long long)nc*nc)), dim3(256), 0, ctx->stream, nc,
-			aug.data(), dinv64.data());
+		hipLaunchKernelGGL(ExtractInverseKernel<double>, dim3(nc), dim3(256), 0, ctx->stream, nc, matrix, pivot.data(),
+			dinv64.data());
 	}
 	TFI_LAUNCH_CHECK("ExtractInverseKernel");
 }
