@@ -285,7 +285,7 @@ struct KrylovResult {
 class Fgmres {
 public:
 	Fgmres(tfi_ctx* ctx, long long n, int restart);
-	// Solves A x = b to ||b - A x|| <= rtol ||b|| (true residual).
+	// Solves A x = b to ||b - A x|| <= rtol ||b|| (true residual); an empty M: no preconditioner.
 	KrylovResult Solve(const Operator& A, const Precond& M, const double* b, double* x, int maxit, double rtol,
 		double absolute_target = 0.0);
 private:

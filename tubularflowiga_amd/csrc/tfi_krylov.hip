@@ -20,8 +20,38 @@ namespace tfi {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPerThread = 8;  // vector entries per thread: eight 8-byte loads per basis vector in flight
-constexpr int kGroup = 8;      // basis vectors per multi-dot pass (one set of wave reductions per pass)
+constexpr int kGroup = 8;         // basis vectors of a multi-dot workgroup (one set of wave reductions)
+constexpr int kMaxPer = 8;        // vector entries per thread, at most
+constexpr int kDotGroups = 2048;  // workgroups of a pass that keep the chip's memory pipes full
+constexpr int kFewBlocks = 32;    // partial sums that the kernel after a multi-dot adds up itself
+
+// Why the split depends on the length: eight entries per thread left 158
+// workgroups for 324,000 entries (25 vectors on average: multi-dot 75 us,
+// multi-axpy 57, 0.9 TB/s) and one for 1800 (20 and 16 us).  With the rule
+// below 13 and 11 us (4.9 TB/s), and 2.8 and 3.9 us; where eight entries per
+// thread already give kDotGroups workgroups nothing changes.
+// Entries per thread of a pass over n entries in `lanes` rows of workgroups: as
+// many as leave kDotGroups workgroups (8-byte loads in flight against workgroups
+// to hide their latency), 1 to kMaxPer.
+int EntriesPerThread(long long n, int lanes)
+{
+	int per = kMaxPer;
+	while (per > 1 && (n + (long long)kThreads*per - 1)/((long long)kThreads*per)*lanes < kDotGroups) per >>= 1;
+	return per;
+}
+int Blocks(long long n, int per)
+{
+	return static_cast<int>((n + (long long)kThreads*per - 1)/((long long)kThreads*per));
+}
+// Most row blocks EntriesPerThread can ask for: below kDotGroups*2 unless every thread has kMaxPer entries
+int MaxBlocks(long long n)
+{
+	return std::min(Blocks(n, 1), std::max(2*kDotGroups, Blocks(n, kMaxPer)));
+}
+// Vectors too short for a workgroup per CU at one entry per thread: the
+// multi-axpy takes 64 entries per workgroup instead
+bool Short(const tfi_ctx* ctx, long long n) { return Blocks(n, 1) < ctx->cus; }
+int ShortBlocks(long long n) { return static_cast<int>((n + 63)/64); }
 
 __device__ inline double WaveSum(double v)
 {
@@ -29,48 +59,60 @@ __device__ inline double WaveSum(double v)
 	return v;
 }
 
-// partial[i*blocks + blk] = sum over this block's rows of V_i . w, i < count.
+// Sums of eight values over the wave: three exchanges halve the values a lane
+// carries while they halve its partners (7 shuffles), three more finish (3):
+// 10 instead of 48.  Lane l ends with the sum of value (l >> 3).
+__device__ inline double WaveSum8(const double (&v)[kGroup])
+{
+	const int lane = threadIdx.x & 63;
+	double a[4], b[2];
+	const bool h32 = lane & 32, h16 = lane & 16, h8 = lane & 8;
+#pragma unroll
+	for (int k = 0; k < 4; ++k) a[k] = (h32 ? v[4 + k] : v[k]) + __shfl_xor(h32 ? v[k] : v[4 + k], 32, 64);
+#pragma unroll
+	for (int k = 0; k < 2; ++k) b[k] = (h16 ? a[2 + k] : a[k]) + __shfl_xor(h16 ? a[k] : a[2 + k], 16, 64);
+	double c = (h8 ? b[1] : b[0]) + __shfl_xor(h8 ? b[0] : b[1], 8, 64);
+	c += __shfl_xor(c, 4, 64);
+	c += __shfl_xor(c, 2, 64);
+	c += __shfl_xor(c, 1, 64);
+	return c;
+}
+
+// partial[i*gridDim.x + blk] = sum over this block's rows of V_i . w, i < count;
+// blockIdx.y: eight of the vectors.
+template <int kPer>
 __global__ void __launch_bounds__(kThreads) MultiDotKernel(const double* __restrict__ V, long long ld, int count,
 	const double* __restrict__ w, long long n, double* __restrict__ partial)
 {
 	__shared__ double lds[kGroup][4];
-	const long long base = (long long)blockIdx.x*kThreads*kPerThread;
-	double wr[kPerThread];
+	const long long base = (long long)blockIdx.x*kThreads*kPer + threadIdx.x;
+	const int g = blockIdx.y*kGroup;
+	double wr[kPer];
 #pragma unroll
-	for (int t = 0; t < kPerThread; ++t) {
-		const long long i = base + (long long)t*kThreads + threadIdx.x;
+	for (int t = 0; t < kPer; ++t) {
+		const long long i = base + (long long)t*kThreads;
 		wr[t] = i < n ? w[i] : 0.0;
 	}
+	double acc[kGroup] = {};
+#pragma unroll
+	for (int v = 0; v < kGroup; ++v) {
+		// past the last vector: its place is read again and not stored
+		const double* Vi = V + (long long)min(g + v, count - 1)*ld;
+#pragma unroll
+		for (int t = 0; t < kPer; ++t) acc[v] += Vi[min(base + (long long)t*kThreads, n - 1)]*wr[t];
+	}
+	const double s = WaveSum8(acc);
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	for (int g = 0; g < count; g += kGroup) {
-		double acc[kGroup] = {};
-#pragma unroll
-		for (int v = 0; v < kGroup; ++v) {
-			if (g + v >= count) break;
-			const double* Vi = V + (long long)(g + v)*ld;
-#pragma unroll
-			for (int t = 0; t < kPerThread; ++t) {
-				const long long i = base + (long long)t*kThreads + threadIdx.x;
-				if (i < n) acc[v] += Vi[i]*wr[t];
-			}
-		}
-#pragma unroll
-		for (int v = 0; v < kGroup; ++v) {
-			const double s = WaveSum(acc[v]);
-			if (lane == 0) lds[v][wave] = s;
-		}
-		__syncthreads();
-		if (threadIdx.x < kGroup && g + (int)threadIdx.x < count) {
-			const int v = threadIdx.x;
-			partial[(long long)(g + v)*gridDim.x + blockIdx.x] = lds[v][0] + lds[v][1] + lds[v][2] + lds[v][3];
-		}
-		__syncthreads();
+	if ((lane & 7) == 0) lds[lane >> 3][wave] = s;
+	__syncthreads();
+	if (threadIdx.x < kGroup && g + (int)threadIdx.x < count) {
+		const int v = threadIdx.x;
+		partial[(long long)(g + v)*gridDim.x + blockIdx.x] = lds[v][0] + lds[v][1] + lds[v][2] + lds[v][3];
 	}
 }
 
-// out[i] = (accumulate ? out[i] : 0) + sum_b partial[i*blocks + b]   (one workgroup per i)
-__global__ void ReducePartialsKernel(const double* __restrict__ partial, int blocks, double* __restrict__ out,
-	int accumulate)
+// out[i] = sum_b partial[i*blocks + b]   (one workgroup per i)
+__global__ void ReducePartialsKernel(const double* __restrict__ partial, int blocks, double* __restrict__ out)
 {
 	__shared__ double lds[4];
 	const int i = blockIdx.x;
@@ -81,61 +123,143 @@ __global__ void ReducePartialsKernel(const double* __restrict__ partial, int blo
 	__syncthreads();
 	if (threadIdx.x == 0) {
 		const double t = lds[0] + lds[1] + lds[2] + lds[3];
-		out[i] = accumulate ? out[i] + t : t;
+		out[i] = t;
 	}
 }
 
-// w += sign * sum_i coef[i] V_i ; optional per-block partial of ||w||^2.
+// w += sign * sum_i coef[i] V_i ; optional per-block partial of ||w||^2.  With
+// partial_blocks > 0 coef[i] is the sum of partial[i*partial_blocks ..] (few
+// blocks), which workgroup 0 also leaves in coef for the host.
+// kSplit = 1: kPer entries per thread; kSplit = 4: 64 entries per workgroup, its
+// four waves a quarter of the vectors each (short vectors: the walk over the
+// vectors is the time).
+template <int kPer, int kSplit>
 __global__ void __launch_bounds__(kThreads) MultiAxpyKernel(const double* __restrict__ V, long long ld, int count,
-	const double* __restrict__ coef, double sign, double* __restrict__ w, long long n, double* __restrict__ norm_partial)
+	double* __restrict__ coef, const double* __restrict__ partial, int partial_blocks, double sign,
+	double* __restrict__ w, long long n, double* __restrict__ norm_partial)
 {
+	static_assert(kSplit == 1 || (kSplit == 4 && kPer == 1), "whole vectors, or quarters of one entry per lane");
 	__shared__ double c[512];
 	__shared__ double lds[4];
-	for (int i = threadIdx.x; i < count; i += kThreads) c[i] = sign*coef[i];
-	__syncthreads();
-	const long long base = (long long)blockIdx.x*kThreads*kPerThread + threadIdx.x;
-	// each entry accumulates over the vectors in order; the thread's entries
-	// are independent, so their loads of one vector are in flight together
-	double acc[kPerThread];
-#pragma unroll
-	for (int t = 0; t < kPerThread; ++t) {
-		const long long i = base + (long long)t*kThreads;
-		acc[t] = i < n ? w[i] : 0.0;
+	for (int i = threadIdx.x; i < count; i += kThreads) {
+		double v;
+		if (partial_blocks > 0) {
+			v = 0.0;
+			for (int b = 0; b < partial_blocks; ++b) v += partial[(long long)i*partial_blocks + b];
+			if (blockIdx.x == 0) coef[i] = v;
+		} else {
+			v = coef[i];
+		}
+		c[i] = sign*v;
 	}
-	for (int v = 0; v < count; ++v) {
+	__syncthreads();
+	const int wave = threadIdx.x >> 6;
+	const long long base = kSplit == 1 ? (long long)blockIdx.x*kThreads*kPer + threadIdx.x
+		: (long long)blockIdx.x*64 + (threadIdx.x & 63);
+	// each entry accumulates over the vectors in order; the loads of eight
+	// vectors are in flight together
+	double acc[kPer];
+#pragma unroll
+	for (int t = 0; t < kPer; ++t) {
+		const long long i = base + (long long)t*kThreads;
+		acc[t] = i < n && (kSplit == 1 || wave == 0) ? w[i] : 0.0;
+	}
+	const int quarter = (count + kSplit - 1)/kSplit;
+	const int begin = kSplit == 1 ? 0 : min(count, wave*quarter), end = kSplit == 1 ? count : min(count, begin + quarter);
+#pragma unroll 8
+	for (int v = begin; v < end; ++v) {
 		const double cv = c[v];
 		const double* Vv = V + (long long)v*ld;
 #pragma unroll
-		for (int t = 0; t < kPerThread; ++t) {
-			const long long i = base + (long long)t*kThreads;
-			if (i < n) acc[t] += cv*Vv[i];
+		for (int t = 0; t < kPer; ++t) acc[t] += cv*Vv[min(base + (long long)t*kThreads, n - 1)];
+	}
+	if constexpr (kSplit > 1) {
+		__shared__ double part[kSplit][64];
+		part[wave][threadIdx.x & 63] = acc[0];
+		__syncthreads();
+		if (wave > 0) {
+			acc[0] = 0.0;  // no share in the norm
+		} else {
+			acc[0] = 0.0;
+			for (int k = 0; k < kSplit; ++k) acc[0] += part[k][threadIdx.x];
 		}
 	}
 	double sq = 0.0;
 #pragma unroll
-	for (int t = 0; t < kPerThread; ++t) {
+	for (int t = 0; t < kPer; ++t) {
 		const long long i = base + (long long)t*kThreads;
-		if (i < n) {
+		if (i < n && (kSplit == 1 || wave == 0)) {
 			w[i] = acc[t];
 			sq += acc[t]*acc[t];
 		}
 	}
 	if (norm_partial) {
 		sq = WaveSum(sq);
-		if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = sq;
+		if ((threadIdx.x & 63) == 0) lds[wave] = sq;
 		__syncthreads();
 		if (threadIdx.x == 0) norm_partial[blockIdx.x] = lds[0] + lds[1] + lds[2] + lds[3];
 	}
 }
 
-// dst = src / norm where norm = sqrt(*sq) (device scalar); writes the norm to *out_norm.
+// dst = src / norm where norm^2 is *sq, or with partial_blocks > 0 the sum of
+// partial[0 .. partial_blocks), which workgroup 0 leaves in *sq.
 __global__ void NormalizeKernel(const double* __restrict__ src, double* __restrict__ dst, long long n,
-	const double* __restrict__ sq)
+	double* __restrict__ sq, const double* __restrict__ partial, int partial_blocks)
 {
-	const double nrm = sqrt(*sq);
+	double total = 0.0;
+	if (partial_blocks > 0) {
+		for (int b = 0; b < partial_blocks; ++b) total += partial[b];
+		if (blockIdx.x == 0 && threadIdx.x == 0) *sq = total;
+	} else {
+		total = *sq;
+	}
+	const double nrm = sqrt(total);
 	const double s = nrm > 1e-300 ? 1.0/nrm : 0.0;
 	for (long long i = blockIdx.x*(long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x*blockDim.x)
 		dst[i] = src[i]*s;
+}
+
+// Launches of the passes: each picks the entries per thread for its length.
+// Returns the number of partial sums per vector.
+int MultiDot(tfi_ctx* ctx, const double* V, long long n, int count, const double* w, double* partial)
+{
+	const int groups = (count + kGroup - 1)/kGroup;
+	const int per = EntriesPerThread(n, groups);
+	const dim3 grid(Blocks(n, per), groups);
+	switch (per) {
+	case 1: hipLaunchKernelGGL(MultiDotKernel<1>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
+	case 2: hipLaunchKernelGGL(MultiDotKernel<2>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
+	case 4: hipLaunchKernelGGL(MultiDotKernel<4>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
+	default: hipLaunchKernelGGL(MultiDotKernel<8>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
+	}
+	TFI_LAUNCH_CHECK("MultiDotKernel");
+	return static_cast<int>(grid.x);
+}
+
+// Coefficients from `blocks` partial sums each (0: they are in coef); returns
+// the number of norm partials written.
+int MultiAxpy(tfi_ctx* ctx, const double* V, long long n, int count, double* coef, const double* partial, int blocks,
+	double sign, double* w, double* norm_partial)
+{
+	if (blocks > kFewBlocks) {
+		hipLaunchKernelGGL(ReducePartialsKernel, dim3(count), dim3(256), 0, ctx->stream, partial, blocks, coef);
+		TFI_LAUNCH_CHECK("ReducePartialsKernel");
+		blocks = 0;
+	}
+	auto launch = [&](auto kernel, int grid) {
+		hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, ctx->stream, V, n, count, coef, partial, blocks, sign,
+			w, n, norm_partial);
+		TFI_LAUNCH_CHECK("MultiAxpyKernel");
+		return grid;
+	};
+	if (Short(ctx, n)) return launch(MultiAxpyKernel<1, 4>, ShortBlocks(n));
+	const int per = EntriesPerThread(n, 1);
+	switch (per) {
+	case 1: return launch(MultiAxpyKernel<1, 1>, Blocks(n, 1));
+	case 2: return launch(MultiAxpyKernel<2, 1>, Blocks(n, 2));
+	case 4: return launch(MultiAxpyKernel<4, 1>, Blocks(n, 4));
+	default: return launch(MultiAxpyKernel<8, 1>, Blocks(n, 8));
+	}
 }
 
 }  // namespace
@@ -147,8 +271,8 @@ Fgmres::Fgmres(tfi_ctx* ctx, long long n, int restart) : ctx_(ctx), n_(n), m_(re
 	Z_.Allocate(ctx, (size_t)m_*n);
 	w_.Allocate(ctx, n);
 	r_.Allocate(ctx, n);
-	const long long blocks = (n + kThreads*kPerThread - 1)/(kThreads*kPerThread);
-	partial_.Allocate(ctx, (size_t)(m_ + 2)*blocks + 8);
+	// multi-dot partials of up to m vectors, then the norm partials of a multi-axpy
+	partial_.Allocate(ctx, (size_t)(m_ + 1)*MaxBlocks(n) + (Short(ctx, n) ? ShortBlocks(n) : MaxBlocks(n)));
 	h_.Allocate(ctx, 2*(m_ + 2) + 8);
 	H_.assign((size_t)(m_ + 1)*m_, 0.0);
 	cs_.assign(m_, 0.0);
@@ -162,7 +286,6 @@ KrylovResult Fgmres::Solve(const Operator& A, const Precond& M, const double* b,
 {
 	tfi_ctx* ctx = ctx_;
 	const long long n = n_;
-	const int blocks = static_cast<int>((n + kThreads*kPerThread - 1)/(kThreads*kPerThread));
 	const int eblocks = static_cast<int>(std::min<long long>((n + 255)/256, 4096));
 	KrylovResult res;
 	res.rhs_norm = Norm2(ctx, b, n);
@@ -199,31 +322,23 @@ KrylovResult Fgmres::Solve(const Operator& A, const Precond& M, const double* b,
 		bool breakdown = false;
 		for (int j = 0; j < m_ && res.iterations < maxit; ++j) {
 			double* vj = V + (long long)j*n;
-			double* zj = Z + (long long)j*n;
-			M(vj, zj);
+			double* zj = M ? Z + (long long)j*n : vj;
+			if (M) M(vj, zj);
 			A(zj, w);
-			// CGS pass 1: h = V^T w ; w -= V h
-			hipLaunchKernelGGL(MultiDotKernel, dim3(blocks), dim3(kThreads), 0, ctx->stream, V, n, j + 1, w, n, partial);
-			TFI_LAUNCH_CHECK("MultiDotKernel");
-			hipLaunchKernelGGL(ReducePartialsKernel, dim3(j + 1), dim3(256), 0, ctx->stream, partial, blocks, h, 0);
-			TFI_LAUNCH_CHECK("ReducePartialsKernel");
-			hipLaunchKernelGGL(MultiAxpyKernel, dim3(blocks), dim3(kThreads), 0, ctx->stream, V, n, j + 1, h, -1.0, w, n,
-				nullptr);
-			TFI_LAUNCH_CHECK("MultiAxpyKernel");
-			// CGS pass 2 (re-orthogonalisation), fused with the norm of w
-			hipLaunchKernelGGL(MultiDotKernel, dim3(blocks), dim3(kThreads), 0, ctx->stream, V, n, j + 1, w, n, partial);
-			TFI_LAUNCH_CHECK("MultiDotKernel");
+			// CGS pass 1: h = V^T w ; w -= V h; pass 2 (re-orthogonalisation) with the norm of w
 			double* h2 = h + (m_ + 2);  // second-pass coefficients
-			hipLaunchKernelGGL(ReducePartialsKernel, dim3(j + 1), dim3(256), 0, ctx->stream, partial, blocks, h2, 0);
-			TFI_LAUNCH_CHECK("ReducePartialsKernel");
-			double* npart = partial + (long long)(m_ + 1)*blocks;
-			hipLaunchKernelGGL(MultiAxpyKernel, dim3(blocks), dim3(kThreads), 0, ctx->stream, V, n, j + 1, h2, -1.0, w,
-				n, npart);
-			TFI_LAUNCH_CHECK("MultiAxpyKernel");
-			hipLaunchKernelGGL(ReducePartialsKernel, dim3(1), dim3(256), 0, ctx->stream, npart, blocks, hsq, 0);
-			TFI_LAUNCH_CHECK("ReducePartialsKernel");
+			double* npart = partial + (long long)(m_ + 1)*MaxBlocks(n);
+			int parts = MultiDot(ctx, V, n, j + 1, w, partial);
+			MultiAxpy(ctx, V, n, j + 1, h, partial, parts, -1.0, w, nullptr);
+			parts = MultiDot(ctx, V, n, j + 1, w, partial);
+			int norms = MultiAxpy(ctx, V, n, j + 1, h2, partial, parts, -1.0, w, npart);
+			if (norms > kFewBlocks) {
+				hipLaunchKernelGGL(ReducePartialsKernel, dim3(1), dim3(256), 0, ctx->stream, npart, norms, hsq);
+				TFI_LAUNCH_CHECK("ReducePartialsKernel");
+				norms = 0;
+			}
 			hipLaunchKernelGGL(NormalizeKernel, dim3(eblocks), dim3(256), 0, ctx->stream, w, V + (long long)(j + 1)*n, n,
-				hsq);
+				hsq, npart, norms);
 			TFI_LAUNCH_CHECK("NormalizeKernel");
 			// bring back h (pass 1 + pass 2) and the squared norm
 			Check(hipMemcpyAsync(hcol, h, sizeof(double)*(2*(m_ + 2)), hipMemcpyDeviceToHost, ctx->stream), "h download");
@@ -262,9 +377,7 @@ KrylovResult Fgmres::Solve(const Operator& A, const Precond& M, const double* b,
 			y_[row] = v/d;
 		}
 		Check(hipMemcpyAsync(h, y_.data(), sizeof(double)*used, hipMemcpyHostToDevice, ctx->stream), "y upload");
-		hipLaunchKernelGGL(MultiAxpyKernel, dim3(blocks), dim3(kThreads), 0, ctx->stream, Z, n, used, h, 1.0, x, n,
-			nullptr);
-		TFI_LAUNCH_CHECK("MultiAxpyKernel update");
+		MultiAxpy(ctx, M ? Z : V, n, used, h, nullptr, 0, 1.0, x, nullptr);
 		beta = true_residual();
 		res.residual = beta;
 		if (beta <= tol) {

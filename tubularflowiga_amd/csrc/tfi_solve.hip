@@ -767,7 +767,7 @@ int tfi_solve_step(tfi_solve* s, int zero_guess, int maximum_iterations, double 
 		else Copy(ctx, s->state.data(), s->next.data(), n);
 		BlockApply(s, s->rhs.data(), s->scaled.data());
 		Operator A = [&](const double* x, double* y) { Spmv(s, s->scaled_left.data(), x, y); };
-		Precond M = [&](const double* v, double* z) { Copy(ctx, v, z, n); };
+		Precond M;  // none beyond the block-Jacobi scaling
 		if (s->preconditioner == TFI_PC_AMG) {
 			if (s->amg_stale) SetupAmg(s);
 			const int N = s->mesh->nodes;

@@ -482,7 +482,7 @@ int tfi_transport_step(tfi_transport* t, int zero_guess, int maximum_iterations,
 		};
 		block_apply(t->rhs.data(), t->scaled.data());
 		Operator A = [&](const double* x, double* y) { Spmv2(t, t->scaled_left.data(), x, y); };
-		Precond M = [&](const double* v, double* z) { Copy(ctx, v, z, n); };
+		Precond M;  // none beyond the block-Jacobi scaling
 		if (t->preconditioner == TFI_PC_AMG) {
 			if (!t->amg) {
 				// the operator is fixed for the run: one AMG set-up (FP32 cycles)
