@@ -10,16 +10,22 @@
 //     the first matrix (field-diagonal couplings), greedy aggregation in node
 //     order, coarse block pattern, and for every coarse block the ascending
 //     list of fine blocks that sum into it;
-//   * numeric phase (GPU, every Newton step): Galerkin coarse blocks as
-//     fixed-order segmented sums (no atomics), 4x4 diagonal inverses, and a
-//     dense Gauss-Jordan inverse of the coarsest operator;
+//   * numeric phase (GPU, every Newton step): A P (the blocks of a row summed
+//     per aggregate of their columns) and from it the Galerkin coarse blocks,
+//     both as fixed-order segmented sums (no atomics), 4x4 diagonal inverses,
+//     and a dense Gauss-Jordan inverse of the coarsest operator;
 //   * V-cycle: symmetric multicolour block Gauss-Seidel (greedy node colouring
 //     per level, one launch per colour, in place -- rows of one colour are
 //     uncoupled), damped block Jacobi with omega = 1.33 / lambda_max(D^-1 A),
 //     or a Chebyshev polynomial in D^-1 A on [0.1, 1.1] lambda_max
 //     (power-iteration estimate; one fused launch per degree, no colours);
 //     restriction = aggregate sums, prolongation = injection; optionally
-//     entirely in FP32.
+//     entirely in FP32.  The first smoothing step after the coarse correction
+//     needs b - A (x + P xc) = r - (A P) xc with the residual r that was
+//     restricted: A P has about a tenth of A's blocks, so that step is not
+//     another pass over A.  With two steps before and after, three passes over
+//     A instead of four: 1624 -> 1264 us in FP64 and 606 -> 499 us with the FP16
+//     smoothing matrices for 16.2 million blocks.
 // The prolongator is the 0/1 aggregate map, stored as integers, so it is exact
 // in any precision.
 #include "tfi_solver.hpp"
@@ -87,7 +93,7 @@ __device__ inline T RowPartial(const int* __restrict__ ro, const int* __restrict
 	return acc;
 }
 
-// x_out = x_in + omega D^-1 (b - A x_in); x_in == nullptr means x_in = 0.
+// x_out = x_in + omega D^-1 (b - A x_in).
 template <class T>
 __global__ void __launch_bounds__(256) SmoothKernel(int rows, const int* __restrict__ ro, const int* __restrict__ cols,
 	const T* __restrict__ vals, const T* __restrict__ inv, const T* __restrict__ b, const T* __restrict__ xin,
@@ -97,27 +103,23 @@ __global__ void __launch_bounds__(256) SmoothKernel(int rows, const int* __restr
 	const int row = blockIdx.x*4 + (threadIdx.x >> 6);
 	if (row >= rows) return;
 	const int sub = lane >> 2, r = lane & 3;
-	T acc = 0;
-	if (xin) {
-		acc = RowPartial(ro, cols, vals, xin, row, sub, r);
-		acc += __shfl_xor(acc, 4, 64);
-		acc += __shfl_xor(acc, 8, 64);
-		acc += __shfl_xor(acc, 16, 64);
-		acc += __shfl_xor(acc, 32, 64);
-	}
+	T acc = RowPartial(ro, cols, vals, xin, row, sub, r);
+	acc += __shfl_xor(acc, 4, 64);
+	acc += __shfl_xor(acc, 8, 64);
+	acc += __shfl_xor(acc, 16, 64);
+	acc += __shfl_xor(acc, 32, 64);
 	// lanes 0..3 hold row residual components after the butterfly
 	const T res = b[4*(size_t)row + r] - acc;
 	const T r0 = __shfl(res, 0, 64), r1 = __shfl(res, 1, 64), r2 = __shfl(res, 2, 64), r3 = __shfl(res, 3, 64);
 	if (sub == 0) {
 		const T* d = inv + (size_t)row*16 + 4*r;
 		const T corr = d[0]*r0 + d[1]*r1 + d[2]*r2 + d[3]*r3;
-		xout[4*(size_t)row + r] = (xin ? xin[4*(size_t)row + r] : T(0)) + omega*corr;
+		xout[4*(size_t)row + r] = xin[4*(size_t)row + r] + omega*corr;
 	}
 }
 
 // One Chebyshev step (three-term form): z = D^-1 (b - A x_in), d = cd d + cz z,
-// x_out = x_in + d; x_in == nullptr means x_in = 0 (and A x_in = 0), cd == 0
-// ignores the old d.  d is per row, so it is updated in place.
+// x_out = x_in + d.  d is per row, so it is updated in place.
 template <class T>
 __global__ void __launch_bounds__(256) ChebyshevKernel(int rows, const int* __restrict__ ro,
 	const int* __restrict__ cols, const T* __restrict__ vals, const T* __restrict__ inv, const T* __restrict__ b,
@@ -127,23 +129,20 @@ __global__ void __launch_bounds__(256) ChebyshevKernel(int rows, const int* __re
 	const int row = blockIdx.x*4 + (threadIdx.x >> 6);
 	if (row >= rows) return;
 	const int sub = lane >> 2, r = lane & 3;
-	T acc = 0;
-	if (xin) {
-		acc = RowPartial(ro, cols, vals, xin, row, sub, r);
-		acc += __shfl_xor(acc, 4, 64);
-		acc += __shfl_xor(acc, 8, 64);
-		acc += __shfl_xor(acc, 16, 64);
-		acc += __shfl_xor(acc, 32, 64);
-	}
+	T acc = RowPartial(ro, cols, vals, xin, row, sub, r);
+	acc += __shfl_xor(acc, 4, 64);
+	acc += __shfl_xor(acc, 8, 64);
+	acc += __shfl_xor(acc, 16, 64);
+	acc += __shfl_xor(acc, 32, 64);
 	const T res = b[4*(size_t)row + r] - acc;
 	const T r0 = __shfl(res, 0, 64), r1 = __shfl(res, 1, 64), r2 = __shfl(res, 2, 64), r3 = __shfl(res, 3, 64);
 	if (sub == 0) {
 		const size_t i = 4*(size_t)row + r;
 		const T* dv = inv + (size_t)row*16 + 4*r;
 		const T z = dv[0]*r0 + dv[1]*r1 + dv[2]*r2 + dv[3]*r3;
-		const T dn = (cd != T(0) ? cd*d[i] : T(0)) + cz*z;
+		const T dn = cd*d[i] + cz*z;
 		d[i] = dn;
-		xout[i] = (xin ? xin[i] : T(0)) + dn;
+		xout[i] = xin[i] + dn;
 	}
 }
 
@@ -200,6 +199,21 @@ __device__ inline float RowProductHalf(const int* __restrict__ ro, const int* __
 	return r == 0 ? a0 : r == 1 ? a1 : r == 2 ? a2 : a3;
 }
 
+// S P: the FP16 blocks of S summed in FP32 over the lists of A P (16 lanes per block)
+__global__ void ScaledGalerkinKernel(long long blocks, const long long* __restrict__ off, const int* __restrict__ list,
+	const _Float16* __restrict__ s, float* __restrict__ out)
+{
+	const long long t = blockIdx.x*(long long)blockDim.x + threadIdx.x;
+	const long long K = t >> 4;
+	if (K >= blocks) return;
+	const int e = t & 15;
+	float v = 0.0f;
+	const long long end = off[K + 1];
+#pragma unroll 4
+	for (long long k = off[K]; k < end; ++k) v += (float)s[(size_t)list[k]*16 + e];
+	out[t] = v;
+}
+
 // S = D^-1 A in FP16 (D^-1 from the FP64 block inverses) and D in FP32; flag
 // set when an entry of S is not finite or above 60000 in magnitude.
 __global__ void __launch_bounds__(256) ScaleBlocksKernel(int rows, const int* __restrict__ ro,
@@ -237,16 +251,15 @@ __global__ void __launch_bounds__(256) ChebyshevScaledKernel(int rows, const int
 	const int row = blockIdx.x*4 + (threadIdx.x >> 6);
 	if (row >= rows) return;
 	const int sub = lane >> 2, r = lane & 3;
-	float acc = 0.0f;
-	if (xin) acc = RowProductHalf(ro, cols, s, xin, row, lane);
+	const float acc = RowProductHalf(ro, cols, s, xin, row, lane);
 	if (sub == 0) {
 		const size_t i = 4*(size_t)row + r;
 		const float* iv = inv + (size_t)row*16 + 4*r;
 		const float* bv = b + 4*(size_t)row;
 		const float z = iv[0]*bv[0] + iv[1]*bv[1] + iv[2]*bv[2] + iv[3]*bv[3] - acc;
-		const float dn = (cd != 0.0f ? cd*d[i] : 0.0f) + cz*z;
+		const float dn = cd*d[i] + cz*z;
 		d[i] = dn;
-		xout[i] = (xin ? xin[i] : 0.0f) + dn;
+		xout[i] = xin[i] + dn;
 	}
 }
 
@@ -335,17 +348,22 @@ __global__ void __launch_bounds__(256) GsColorKernel(int count, const int* __res
 	}
 }
 
-// bc[I] = sum_{i in aggregate I} r[i] (ascending fine order)
+// bc[I] = sum_{i in aggregate I} r[i]: 16 lanes per aggregate, lane (m, c)
+// every fourth member's component c (one lane per component walked the 20 to 30
+// members one after the other: 15 us for 150,000 rows, whatever their bytes)
 template <class T>
-__global__ void RestrictKernel(int coarse, const int* __restrict__ aoff, const int* __restrict__ amem,
-	const T* __restrict__ r, T* __restrict__ bc)
+__global__ void __launch_bounds__(256) RestrictKernel(int coarse, const int* __restrict__ aoff,
+	const int* __restrict__ amem, const T* __restrict__ r, T* __restrict__ bc)
 {
 	const int t = blockIdx.x*blockDim.x + threadIdx.x;
-	const int I = t >> 2, c = t & 3;
-	if (I >= coarse) return;
+	const int I = t >> 4, m = (t >> 2) & 3, c = t & 3;
 	T s = 0;
-	for (int k = aoff[I]; k < aoff[I + 1]; ++k) s += r[4*(size_t)amem[k] + c];
-	bc[4*(size_t)I + c] = s;
+	if (I < coarse)
+#pragma unroll 4
+		for (int k = aoff[I] + m; k < aoff[I + 1]; k += 4) s += r[4*(size_t)amem[k] + c];
+	s += __shfl_xor(s, 4, 64);
+	s += __shfl_xor(s, 8, 64);
+	if (I < coarse && m == 0) bc[4*(size_t)I + c] = s;
 }
 
 // x[i] += xc[agg[i]]
@@ -358,7 +376,55 @@ __global__ void ProlongKernel(int fine, const int* __restrict__ agg, const T* __
 	x[4*(size_t)i + c] += xc[4*(size_t)agg[i] + c];
 }
 
-// coarse[K] = sum of fine blocks list[off[K]..off[K+1]) (16 lanes per block)
+// First smoothing step from x = 0: d = cz D^-1 b, x = d.
+template <class T>
+__global__ void FirstStepKernel(int rows, const T* __restrict__ inv, const T* __restrict__ b, T* __restrict__ x,
+	T* __restrict__ d, T cz)
+{
+	const int t = blockIdx.x*blockDim.x + threadIdx.x;
+	const int row = t >> 2;
+	if (row >= rows) return;
+	const T* dv = inv + 4*(size_t)t;
+	const T* bv = b + 4*(size_t)row;
+	const T v = cz*(dv[0]*bv[0] + dv[1]*bv[1] + dv[2]*bv[2] + dv[3]*bv[3]);
+	d[t] = v;
+	x[t] = v;
+}
+
+// Coarse correction and first smoothing step after it: with A P xc from the
+// row's blocks of A P, d = cz D^-1 (r - A P xc) and x += xc[agg] + d, in place;
+// d takes the place of r.  kScaled: ap holds S P, S = D^-1 A as the level's other
+// steps read it, and d = cz (D^-1 r - S P xc).
+template <class T, bool kScaled>
+__global__ void __launch_bounds__(256) CorrectStepKernel(int rows, const int* __restrict__ ro,
+	const int* __restrict__ cols, const T* __restrict__ ap, const T* __restrict__ inv, const int* __restrict__ agg,
+	const T* __restrict__ xc, T* __restrict__ x, T* __restrict__ rd, T cz)
+{
+	const int lane = threadIdx.x & 63;
+	const int row = blockIdx.x*4 + (threadIdx.x >> 6);
+	if (row >= rows) return;
+	const int sub = lane >> 2, r = lane & 3;
+	T acc = RowPartial(ro, cols, ap, xc, row, sub, r);
+	acc += __shfl_xor(acc, 4, 64);
+	acc += __shfl_xor(acc, 8, 64);
+	acc += __shfl_xor(acc, 16, 64);
+	acc += __shfl_xor(acc, 32, 64);
+	const size_t i = 4*(size_t)row + r;
+	const T res = kScaled ? rd[i] : rd[i] - acc;
+	const T r0 = __shfl(res, 0, 64), r1 = __shfl(res, 1, 64), r2 = __shfl(res, 2, 64), r3 = __shfl(res, 3, 64);
+	if (sub == 0) {
+		const T* dv = inv + (size_t)row*16 + 4*r;
+		T z = dv[0]*r0 + dv[1]*r1 + dv[2]*r2 + dv[3]*r3;
+		if (kScaled) z -= acc;
+		const T d = cz*z;
+		rd[i] = d;
+		x[i] += xc[4*(size_t)agg[row] + r] + d;
+	}
+}
+
+// coarse[K] = sum of fine blocks list[off[K]..off[K+1]) (16 lanes per block): A P from A, the coarse
+// blocks from A P (from A itself, in one gather, each block's list spans rows far apart: 760 against
+// 430 us for 16.2 million blocks)
 __global__ void GalerkinKernel(long long cblocks, const long long* __restrict__ off, const int* __restrict__ list,
 	const double* __restrict__ fine, double* __restrict__ coarse)
 {
@@ -367,7 +433,9 @@ __global__ void GalerkinKernel(long long cblocks, const long long* __restrict__ 
 	const int e = t & 15;
 	if (K >= cblocks) return;
 	double s = 0.0;
-	for (long long k = off[K]; k < off[K + 1]; ++k) s += fine[(size_t)list[k]*16 + e];
+	const long long end = off[K + 1];
+#pragma unroll 4
+	for (long long k = off[K]; k < end; ++k) s += fine[(size_t)list[k]*16 + e];
 	coarse[(size_t)K*16 + e] = s;
 }
 
@@ -595,7 +663,13 @@ struct Level {
 	bool scaled = false;
 	// transfer to the next level
 	DevBuf<int> agg, aoff, amem;
-	DevBuf<long long> goff;       // Galerkin lists for the NEXT level's blocks
+	// A P: its pattern, the fine blocks of each of its blocks, its values
+	DevBuf<int> ap_ro, ap_cols, ap_list;
+	DevBuf<long long> ap_off;
+	DevBuf<double> ap64;
+	DevBuf<float> ap32;
+	long long ap_nnzb = 0;
+	DevBuf<long long> goff;       // the blocks of A P of each block of the NEXT level
 	DevBuf<int> glist;
 	// multicolour Gauss-Seidel (gs) or damped block Jacobi; rows grouped by colour
 	bool gs = false;
@@ -625,7 +699,8 @@ struct Amg::Impl {
 	void Numeric(const double* fine_values64, const float* fine_values32);
 	void Colour(Level& v);
 	template <class T>
-	void Cycle(int l);
+	void Cycle(int l, const T* b, T* x);
+	void Coarsen(Level& fine, const double* fine_values, Level& coarse);
 };
 
 namespace {
@@ -780,60 +855,95 @@ void Amg::Impl::Symbolic(const double* fine_values)
 			std::vector<int> fill(aoff.begin(), aoff.end() - 1);
 			for (int i = 0; i < f.rows; ++i) amem[fill[agg[i]]++] = i;
 		}
-		// coarse pattern
+		// pattern of A P: the aggregates of each row's columns, ascending; the
+		// fine blocks of each of its blocks, ascending
+		std::vector<int> ap_ro(f.rows + 1, 0), ap_cols, ap_list(f.nnzb), touched, place(count, -1);
+		std::vector<long long> ap_off(1, 0);
+		ap_cols.reserve(f.nnzb/4);
+		ap_off.reserve(f.nnzb/4);
+		std::vector<int> fill;
+		for (int i = 0; i < f.rows; ++i) {
+			const int begin = f.h_ro[i], end = f.h_ro[i + 1];
+			touched.clear();
+			for (int k = begin; k < end; ++k) {
+				const int J = agg[f.h_cols[k]];
+				if (place[J] < 0) {
+					place[J] = 0;
+					touched.push_back(J);
+				}
+				++place[J];
+			}
+			std::sort(touched.begin(), touched.end());
+			fill.clear();
+			for (int J : touched) {
+				const int members = place[J];
+				place[J] = static_cast<int>(fill.size());
+				fill.push_back(static_cast<int>(ap_off.back()));
+				ap_cols.push_back(J);
+				ap_off.push_back(ap_off.back() + members);
+			}
+			for (int k = begin; k < end; ++k) ap_list[fill[place[agg[f.h_cols[k]]]]++] = k;
+			for (int J : touched) place[J] = -1;
+			ap_ro[i + 1] = static_cast<int>(ap_cols.size());
+		}
+		f.ap_nnzb = ap_ro[f.rows];
+		// coarse pattern: the union of the rows of A P of an aggregate's members; the
+		// blocks of A P of each coarse block in the order of the members
 		auto c = std::make_unique<Level>();
 		c->rows = count;
-		std::vector<std::vector<int>> rows(count);
-		for (int i = 0; i < f.rows; ++i) {
-			auto& rw = rows[agg[i]];
-			for (int k = f.h_ro[i]; k < f.h_ro[i + 1]; ++k) rw.push_back(agg[f.h_cols[k]]);
-		}
 		c->h_ro.assign(count + 1, 0);
 		c->h_diag.assign(count, -1);
+		std::vector<int> list(f.ap_nnzb);
+		std::vector<long long> cnt(1, 0);
+		long long written = 0;
 		for (int I = 0; I < count; ++I) {
-			auto& rw = rows[I];
-			std::sort(rw.begin(), rw.end());
-			rw.erase(std::unique(rw.begin(), rw.end()), rw.end());
-			c->h_ro[I + 1] = c->h_ro[I] + static_cast<int>(rw.size());
-		}
-		c->nnzb = c->h_ro[count];
-		c->h_cols.resize(c->nnzb);
-		for (int I = 0; I < count; ++I) {
-			std::copy(rows[I].begin(), rows[I].end(), c->h_cols.begin() + c->h_ro[I]);
-			const auto it = std::lower_bound(rows[I].begin(), rows[I].end(), I);
-			c->h_diag[I] = c->h_ro[I] + static_cast<int>(it - rows[I].begin());
-			std::vector<int>().swap(rows[I]);
-		}
-		// fine block -> coarse block lists (ascending fine block index)
-		std::vector<long long> cnt(c->nnzb + 1, 0);
-		std::vector<int> target(f.nnzb);
-		for (int i = 0; i < f.rows; ++i) {
-			const int I = agg[i];
-			const int* b = c->h_cols.data() + c->h_ro[I];
-			const int* e = c->h_cols.data() + c->h_ro[I + 1];
-			for (int k = f.h_ro[i]; k < f.h_ro[i + 1]; ++k) {
-				const int J = agg[f.h_cols[k]];
-				const int pos = static_cast<int>(std::lower_bound(b, e, J) - c->h_cols.data());
-				target[k] = pos;
-				++cnt[pos + 1];
+			touched.clear();
+			for (int m = aoff[I]; m < aoff[I + 1]; ++m)
+				for (int k = ap_ro[amem[m]]; k < ap_ro[amem[m] + 1]; ++k) {
+					const int J = ap_cols[k];
+					if (place[J] < 0) {
+						place[J] = 0;
+						touched.push_back(J);
+					}
+					++place[J];
+				}
+			std::sort(touched.begin(), touched.end());
+			fill.clear();
+			for (int J : touched) {
+				const int members = place[J];
+				place[J] = static_cast<int>(fill.size());
+				fill.push_back(static_cast<int>(cnt.back()));
+				if (J == I) c->h_diag[I] = static_cast<int>(written);
+				c->h_cols.push_back(J);
+				cnt.push_back(cnt.back() + members);
+				++written;
 			}
+			for (int m = aoff[I]; m < aoff[I + 1]; ++m)
+				for (int k = ap_ro[amem[m]]; k < ap_ro[amem[m] + 1]; ++k) list[fill[place[ap_cols[k]]]++] = k;
+			for (int J : touched) place[J] = -1;
+			c->h_ro[I + 1] = static_cast<int>(written);
 		}
-		for (long long K = 0; K < c->nnzb; ++K) cnt[K + 1] += cnt[K];
-		std::vector<int> list(f.nnzb);
-		{
-			std::vector<long long> fill(cnt.begin(), cnt.end() - 1);
-			for (long long k = 0; k < f.nnzb; ++k) list[fill[target[k]]++] = static_cast<int>(k);
-		}
+		c->nnzb = written;
 		f.agg.Allocate(ctx, f.rows);
 		f.agg.Upload(agg.data(), f.rows);
 		f.aoff.Allocate(ctx, count + 1);
 		f.aoff.Upload(aoff.data(), count + 1);
 		f.amem.Allocate(ctx, f.rows);
 		f.amem.Upload(amem.data(), f.rows);
+		f.ap_ro.Allocate(ctx, f.rows + 1);
+		f.ap_ro.Upload(ap_ro.data(), f.rows + 1);
+		f.ap_cols.Allocate(ctx, f.ap_nnzb);
+		f.ap_cols.Upload(ap_cols.data(), f.ap_nnzb);
+		f.ap_off.Allocate(ctx, f.ap_nnzb + 1);
+		f.ap_off.Upload(ap_off.data(), f.ap_nnzb + 1);
+		f.ap_list.Allocate(ctx, f.nnzb);
+		f.ap_list.Upload(ap_list.data(), f.nnzb);
+		f.ap64.Allocate(ctx, f.ap_nnzb*16);
+		if (precision == TFI_MIXED) f.ap32.Allocate(ctx, f.ap_nnzb*16);
 		f.goff.Allocate(ctx, c->nnzb + 1);
 		f.goff.Upload(cnt.data(), c->nnzb + 1);
-		f.glist.Allocate(ctx, f.nnzb);
-		f.glist.Upload(list.data(), f.nnzb);
+		f.glist.Allocate(ctx, f.ap_nnzb);
+		f.glist.Upload(list.data(), f.ap_nnzb);
 		c->ro_own.Allocate(ctx, count + 1);
 		c->ro_own.Upload(c->h_ro.data(), count + 1);
 		c->cols_own.Allocate(ctx, c->nnzb);
@@ -845,9 +955,7 @@ void Amg::Impl::Symbolic(const double* fine_values)
 		c->diag = c->diag_own.data();
 		c->vals.Allocate(ctx, c->nnzb*16);
 		// coarse values now (the next aggregation needs them)
-		hipLaunchKernelGGL(GalerkinKernel, dim3(Grid(c->nnzb*16)), dim3(256), 0, ctx->stream, c->nnzb, f.goff.data(),
-			f.glist.data(), L.size() == 1 ? fine_values : f.vals.data(), c->vals.data());
-		TFI_LAUNCH_CHECK("GalerkinKernel");
+		Coarsen(f, L.size() == 1 ? fine_values : f.vals.data(), *c);
 		hv.assign(c->nnzb*16, 0.0);
 		c->vals.Download(hv.data(), hv.size());
 		L.push_back(std::move(c));
@@ -871,9 +979,11 @@ void Amg::Impl::Symbolic(const double* fine_values)
 				v.dblock32.Allocate(ctx, 16LL*v.rows);
 			}
 		} else {
-			v.x64.Allocate(ctx, n);
+			if (l > 0) {  // the finest level works on the caller's vectors
+				v.x64.Allocate(ctx, n);
+				v.b64.Allocate(ctx, n);
+			}
 			v.y64.Allocate(ctx, n);
-			v.b64.Allocate(ctx, n);
 			v.r64.Allocate(ctx, n);
 		}
 	}
@@ -891,6 +1001,17 @@ void Amg::Impl::Symbolic(const double* fine_values)
 	built = true;
 }
 
+// A P of the fine level, then the coarse values from it
+void Amg::Impl::Coarsen(Level& f, const double* fine_values, Level& c)
+{
+	hipLaunchKernelGGL(GalerkinKernel, dim3(Grid(f.ap_nnzb*16)), dim3(256), 0, ctx->stream, f.ap_nnzb, f.ap_off.data(),
+		f.ap_list.data(), fine_values, f.ap64.data());
+	TFI_LAUNCH_CHECK("GalerkinKernel A P");
+	hipLaunchKernelGGL(GalerkinKernel, dim3(Grid(c.nnzb*16)), dim3(256), 0, ctx->stream, c.nnzb, f.goff.data(),
+		f.glist.data(), f.ap64.data(), c.vals.data());
+	TFI_LAUNCH_CHECK("GalerkinKernel");
+}
+
 void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 {
 	L[0]->vals64 = fine64;
@@ -898,9 +1019,7 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 	for (size_t l = 0; l + 1 < L.size(); ++l) {
 		Level& f = *L[l];
 		Level& c = *L[l + 1];
-		hipLaunchKernelGGL(GalerkinKernel, dim3(Grid(c.nnzb*16)), dim3(256), 0, ctx->stream, c.nnzb, f.goff.data(),
-			f.glist.data(), l == 0 ? fine64 : f.vals.data(), c.vals.data());
-		TFI_LAUNCH_CHECK("GalerkinKernel");
+		Coarsen(f, l == 0 ? fine64 : f.vals.data(), c);
 		c.vals64 = c.vals.data();
 	}
 	for (size_t l = 0; l < L.size(); ++l) {
@@ -934,6 +1053,18 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 		scale_flags.Download(flags.data(), flags.size());
 		for (size_t l = 0; l < L.size(); ++l) L[l]->scaled = L[l]->s16.size() > 0 && !L[l]->gs && flags[l] == 0;
 	}
+	// FP32 A P, or S P where the level's steps read S
+	if (precision == TFI_MIXED)
+		for (size_t l = 0; l + 1 < L.size(); ++l) {
+			Level& v = *L[l];
+			if (v.scaled)
+				hipLaunchKernelGGL(ScaledGalerkinKernel, dim3(Grid(v.ap_nnzb*16)), dim3(256), 0, ctx->stream, v.ap_nnzb,
+					v.ap_off.data(), v.ap_list.data(), v.s16.data(), v.ap32.data());
+			else if (!v.gs)
+				hipLaunchKernelGGL(ToFloatKernel2, dim3(Grid(std::min<long long>(v.ap_nnzb*16, 1LL << 22))), dim3(256), 0,
+					ctx->stream, v.ap_nnzb*16, v.ap64.data(), v.ap32.data());
+			TFI_LAUNCH_CHECK("FP32 A P");
+		}
 	// lambda_max(D^-1 A) of every Jacobi-smoothed level by power iteration (FP64)
 	for (size_t l = 0; l + 1 < L.size(); ++l) {
 			Level& v = *L[l];
@@ -986,57 +1117,67 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 	TFI_LAUNCH_CHECK("ExtractInverseKernel");
 }
 
+// x = M^-1 b on level l
 template <class T>
-void Amg::Impl::Cycle(int l)
+void Amg::Impl::Cycle(int l, const T* b, T* x)
 {
 	Level& v = *L[l];
-	const bool f32 = std::is_same<T, float>::value;
-	T* x = f32 ? reinterpret_cast<T*>(v.x32.data()) : reinterpret_cast<T*>(v.x64.data());
-	T* y = f32 ? reinterpret_cast<T*>(v.y32.data()) : reinterpret_cast<T*>(v.y64.data());
-	T* b = f32 ? reinterpret_cast<T*>(v.b32.data()) : reinterpret_cast<T*>(v.b64.data());
-	T* r = f32 ? reinterpret_cast<T*>(v.r32.data()) : reinterpret_cast<T*>(v.r64.data());
-	const T* vals = f32 ? reinterpret_cast<const T*>(v.vals32) : reinterpret_cast<const T*>(v.vals64);
-	const T* inv = f32 ? reinterpret_cast<const T*>(v.inv32.data()) : reinterpret_cast<const T*>(v.inv64.data());
-	const int grid = (v.rows + 3)/4;
+	constexpr bool f32 = std::is_same<T, float>::value;
+	auto pick = [](auto& wide, auto& narrow) -> T* {
+		if constexpr (f32) return narrow.data();
+		else return wide.data();
+	};
 	if (l + 1 == (int)L.size()) {
-		const T* dinv = f32 ? reinterpret_cast<const T*>(dinv32.data()) : reinterpret_cast<const T*>(dinv64.data());
-		hipLaunchKernelGGL(DenseApplyKernel<T>, dim3((nc + 3)/4), dim3(256), 0, ctx->stream, nc, dinv, b, x);
+		hipLaunchKernelGGL(DenseApplyKernel<T>, dim3((nc + 3)/4), dim3(256), 0, ctx->stream, nc,
+			static_cast<const T*>(pick(dinv64, dinv32)), b, x);
 		TFI_LAUNCH_CHECK("DenseApplyKernel");
 		return;
 	}
-	const T omega = static_cast<T>(kOmegaScale/v.lambda_max);
+	T* y = pick(v.y64, v.y32);
+	T* r = pick(v.r64, v.r32);
+	const T* vals;
+	if constexpr (f32) vals = v.vals32;
+	else vals = v.vals64;
+	const T* inv = pick(v.inv64, v.inv32);
+	const int grid = (v.rows + 3)/4;
 	const bool gs = v.gs;
 	const bool cheb = !gs && opt.smoother == TFI_SMOOTH_CHEBYSHEV;
-	// Chebyshev steps on [kChebLow, kChebHigh] lambda_max from x (x_in == nullptr: from 0);
-	// d lives in the level's r buffer, which the smoothing phases do not otherwise use
-	auto chebyshev = [&](int degree, bool from_zero) {
-		const double hi = kChebHigh*v.lambda_max, lo = kChebLow*v.lambda_max;
-		const double theta = 0.5*(hi + lo), delta = 0.5*(hi - lo), sigma = theta/delta;
+	// Smoothing steps before and after the coarse correction.  The first of
+	// either needs no pass over A: from x = 0, or from the residual and A P; the
+	// others go from x to y and back, and their number before and after is the
+	// same, so the result is in x.  Chebyshev steps on [kChebLow, kChebHigh]
+	// lambda_max: d lives in the level's r buffer, which the smoothing phases do
+	// not otherwise use.
+	const int steps = cheb ? opt.chebyshev_degree : kPre;
+	static_assert(kPre == kPost, "as many steps after the correction as before");
+	const double hi = kChebHigh*v.lambda_max, lo = kChebLow*v.lambda_max;
+	const double theta = 0.5*(hi + lo), delta = 0.5*(hi - lo), sigma = theta/delta;
+	const T first = static_cast<T>(cheb ? 1.0/theta : kOmegaScale/v.lambda_max);
+	T* from = x;
+	T* to = y;
+	auto more_steps = [&] {
 		double rho = 1.0/sigma;
-		for (int k = 0; k < degree; ++k) {
-			double cd = 0.0, cz = 1.0/theta;
-			if (k > 0) {
-				const double rn = 1.0/(2.0*sigma - rho);
-				cd = rn*rho;
-				cz = 2.0*rn/delta;
-				rho = rn;
-			}
+		for (int k = 1; k < steps; ++k) {
+			const double rn = 1.0/(2.0*sigma - rho);
+			const T cd = static_cast<T>(rn*rho), cz = static_cast<T>(2.0*rn/delta);
+			rho = rn;
 			bool done = false;
-			if constexpr (std::is_same<T, float>::value) {
-				if (v.scaled) {
+			if constexpr (f32) {
+				if (cheb && v.scaled) {
 					hipLaunchKernelGGL(ChebyshevScaledKernel, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols,
-						v.s16.data(), inv, b, (k == 0 && from_zero) ? static_cast<const float*>(nullptr) : x, y, r,
-						static_cast<float>(cd), static_cast<float>(cz));
+						v.s16.data(), inv, b, static_cast<const float*>(from), to, r, cd, cz);
 					done = true;
 				}
 			}
-			if (!done)
+			if (!done && cheb)
 				hipLaunchKernelGGL(ChebyshevKernel<T>, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, vals,
-					inv, b, (k == 0 && from_zero) ? static_cast<const T*>(nullptr) : static_cast<const T*>(x), y, r,
-					static_cast<T>(cd), static_cast<T>(cz));
-			std::swap(x, y);
+					inv, b, static_cast<const T*>(from), to, r, cd, cz);
+			else if (!done)
+				hipLaunchKernelGGL(SmoothKernel<T>, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, vals, inv,
+					b, static_cast<const T*>(from), to, first);
+			std::swap(from, to);
 		}
-		TFI_LAUNCH_CHECK("ChebyshevKernel");
+		TFI_LAUNCH_CHECK("smoothing step");
 	};
 	const int ncol = static_cast<int>(v.color_offsets.size()) - 1;
 	// after_forward: this backward sweep directly follows a forward one, whose
@@ -1060,67 +1201,50 @@ void Amg::Impl::Cycle(int l)
 	if (gs) {
 		// symmetric multicolour Gauss-Seidel from x = 0
 		const long long n = 4LL*v.rows;
-		if (f32) Check(hipMemsetAsync(x, 0, n*sizeof(T), ctx->stream), "memset");
-		else Fill(ctx, reinterpret_cast<double*>(x), 0.0, n);
+		if constexpr (f32) Check(hipMemsetAsync(x, 0, n*sizeof(T), ctx->stream), "memset");
+		else Fill(ctx, x, 0.0, n);
 		gs_sweep(true);
 		if (opt.gs_sweeps > 1) gs_sweep(false, true);
-	} else if (cheb) {
-		chebyshev(opt.chebyshev_degree, true);
 	} else {
-		// damped block Jacobi from x = 0
-		hipLaunchKernelGGL(SmoothKernel<T>, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, vals, inv, b,
-			static_cast<const T*>(nullptr), x, omega);
-		for (int s = 1; s < kPre; ++s) {
-			hipLaunchKernelGGL(SmoothKernel<T>, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, vals, inv,
-				b, x, y, omega);
-			std::swap(x, y);
-		}
+		hipLaunchKernelGGL(FirstStepKernel<T>, dim3(Grid(4LL*v.rows)), dim3(256), 0, ctx->stream, v.rows, inv, b, from, r,
+			first);
+		TFI_LAUNCH_CHECK("FirstStepKernel");
+		more_steps();
 	}
 	bool residual_done = false;
-	if constexpr (std::is_same<T, float>::value) {
+	if constexpr (f32) {
 		if (cheb && v.scaled) {
 			hipLaunchKernelGGL(ResidualScaledKernel, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols,
-				v.s16.data(), inv, v.dblock32.data(), b, x, r);
+				v.s16.data(), inv, v.dblock32.data(), b, static_cast<const float*>(from), r);
 			residual_done = true;
 		}
 	}
 	if (!residual_done)
-		hipLaunchKernelGGL(ResidualKernel<T>, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, vals, b, x, r);
+		hipLaunchKernelGGL(ResidualKernel<T>, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, vals, b,
+			static_cast<const T*>(from), r);
 	TFI_LAUNCH_CHECK("ResidualKernel");
 	Level& c = *L[l + 1];
-	T* bc = f32 ? reinterpret_cast<T*>(c.b32.data()) : reinterpret_cast<T*>(c.b64.data());
-	T* xc = f32 ? reinterpret_cast<T*>(c.x32.data()) : reinterpret_cast<T*>(c.x64.data());
-	hipLaunchKernelGGL(RestrictKernel<T>, dim3(Grid(4LL*c.rows)), dim3(256), 0, ctx->stream, c.rows, v.aoff.data(),
-		v.amem.data(), r, bc);
+	T* bc = pick(c.b64, c.b32);
+	T* xc = pick(c.x64, c.x32);
+	hipLaunchKernelGGL(RestrictKernel<T>, dim3(Grid(16LL*c.rows)), dim3(256), 0, ctx->stream, c.rows, v.aoff.data(),
+		v.amem.data(), static_cast<const T*>(r), bc);
 	TFI_LAUNCH_CHECK("RestrictKernel");
-	Cycle<T>(l + 1);
-	// the coarse solution lives in c.x (cycle output); when the coarse cycle
-	// ended with an odd number of swaps it is in c.y -- Cycle always leaves it in x
-	hipLaunchKernelGGL(ProlongKernel<T>, dim3(Grid(4LL*v.rows)), dim3(256), 0, ctx->stream, v.rows, v.agg.data(), xc,
-		x);
-	TFI_LAUNCH_CHECK("ProlongKernel");
+	Cycle<T>(l + 1, bc, xc);
 	if (gs) {
+		hipLaunchKernelGGL(ProlongKernel<T>, dim3(Grid(4LL*v.rows)), dim3(256), 0, ctx->stream, v.rows, v.agg.data(),
+			static_cast<const T*>(xc), x);
+		TFI_LAUNCH_CHECK("ProlongKernel");
 		if (opt.gs_sweeps > 1) gs_sweep(true);
 		gs_sweep(false, opt.gs_sweeps > 1);
-	} else if (cheb) {
-		chebyshev(opt.chebyshev_degree, false);
 	} else {
-		for (int s = 0; s < kPost; ++s) {
-			hipLaunchKernelGGL(SmoothKernel<T>, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, vals, inv,
-				b, x, y, omega);
-			std::swap(x, y);
-		}
-	}
-	TFI_LAUNCH_CHECK("SmoothKernel");
-	// leave the result in the level's x buffer
-	T* xbuf = f32 ? reinterpret_cast<T*>(v.x32.data()) : reinterpret_cast<T*>(v.x64.data());
-	if (x != xbuf) {
-		const long long n = 4LL*v.rows;
-		if (f32) {
-			Check(hipMemcpyAsync(xbuf, x, n*sizeof(T), hipMemcpyDeviceToDevice, ctx->stream), "copy");
-		} else {
-			Copy(ctx, reinterpret_cast<const double*>(x), reinterpret_cast<double*>(xbuf), n);
-		}
+		auto correct = [&](auto kernel) {
+			hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ap_ro.data(), v.ap_cols.data(),
+				static_cast<const T*>(pick(v.ap64, v.ap32)), inv, v.agg.data(), static_cast<const T*>(xc), from, r, first);
+		};
+		if (f32 && cheb && v.scaled) correct(CorrectStepKernel<T, f32>);
+		else correct(CorrectStepKernel<T, false>);
+		TFI_LAUNCH_CHECK("CorrectStepKernel");
+		more_steps();
 	}
 }
 
@@ -1179,13 +1303,16 @@ void Amg::Apply(const double* v, double* z)
 	if (I.precision == TFI_MIXED) {
 		hipLaunchKernelGGL(ToFloatKernel2, dim3(Grid(n)), dim3(256), 0, I.ctx->stream, n, v, l0.b32.data());
 		TFI_LAUNCH_CHECK("ToFloatKernel2");
-		I.Cycle<float>(0);
+		I.Cycle<float>(0, l0.b32.data(), l0.x32.data());
 		hipLaunchKernelGGL(ToDoubleKernel, dim3(Grid(n)), dim3(256), 0, I.ctx->stream, n, l0.x32.data(), z);
 		TFI_LAUNCH_CHECK("ToDoubleKernel");
 	} else {
-		Copy(I.ctx, v, l0.b64.data(), n);
-		I.Cycle<double>(0);
-		Copy(I.ctx, l0.x64.data(), z, n);
+		if (v < z + n && z < v + n) {  // the cycle writes z while it still reads v
+			if (!l0.b64.size()) l0.b64.Allocate(I.ctx, n);
+			Copy(I.ctx, v, l0.b64.data(), n);
+			v = l0.b64.data();
+		}
+		I.Cycle<double>(0, v, z);
 	}
 }
 
