@@ -44,6 +44,7 @@ constexpr double kOmegaScale = 1.33;   // block-Jacobi damping = kOmegaScale / l
 constexpr int kPre = 2, kPost = 2;      // Jacobi sweeps / Chebyshev degree
 constexpr double kChebLow = 0.1, kChebHigh = 1.1;  // Chebyshev interval, in units of lambda_max(D^-1 A)
 constexpr int kPowerIterations = 12;
+constexpr int kPowerBlocks = 4096;     // workgroups of a power-iteration product, at most
 
 template <class T>
 __device__ inline T WaveSumT(T v)
@@ -284,42 +285,69 @@ __global__ void __launch_bounds__(256) ResidualScaledKernel(int rows, const int*
 	}
 }
 
-// y = D^-1 (A x)  (power iteration for lambda_max of the Jacobi-preconditioned operator)
+// Power iteration for lambda_max of the Jacobi-preconditioned operator, without
+// a host in the loop: y = D^-1 A x / sqrt(*sq) with sq = ||x||^2 from the step
+// before, and per workgroup the sum of the squares of its y.  (With the norms
+// read back to the host a step of 42,000 rows took 96 us for 54 us of product.)
 __global__ void __launch_bounds__(256) DinvAKernel(int rows, const int* __restrict__ ro, const int* __restrict__ cols,
 	const double* __restrict__ vals, const double* __restrict__ inv, const double* __restrict__ x,
-	double* __restrict__ y)
+	const double* __restrict__ sq, double* __restrict__ y, double* __restrict__ partial)
 {
-	const int lane = threadIdx.x & 63;
-	const int row = blockIdx.x*4 + (threadIdx.x >> 6);
-	if (row >= rows) return;
+	__shared__ double lds[4];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int sub = lane >> 2, r = lane & 3;
-	double acc = 0.0;
-	for (int k = ro[row] + sub; k < ro[row + 1]; k += 16) {
-		const double* a = vals + (size_t)k*16 + 4*r;
-		const double* xv = x + 4*(size_t)cols[k];
-		acc += a[0]*xv[0] + a[1]*xv[1] + a[2]*xv[2] + a[3]*xv[3];
+	const double scale = 1.0/sqrt(*sq);
+	double total = 0.0;
+	for (int row = blockIdx.x*4 + wave; row < rows; row += 4*gridDim.x) {
+		double acc = RowPartial(ro, cols, vals, x, row, sub, r);
+		acc += __shfl_xor(acc, 4, 64);
+		acc += __shfl_xor(acc, 8, 64);
+		acc += __shfl_xor(acc, 16, 64);
+		acc += __shfl_xor(acc, 32, 64);
+		const double a0 = __shfl(acc, 0, 64), a1 = __shfl(acc, 1, 64), a2 = __shfl(acc, 2, 64), a3 = __shfl(acc, 3, 64);
+		if (sub == 0) {
+			const double* d = inv + (size_t)row*16 + 4*r;
+			const double v = scale*(d[0]*a0 + d[1]*a1 + d[2]*a2 + d[3]*a3);
+			y[4*(size_t)row + r] = v;
+			total += v*v;
+		}
 	}
-	acc += __shfl_xor(acc, 4, 64);
-	acc += __shfl_xor(acc, 8, 64);
-	acc += __shfl_xor(acc, 16, 64);
-	acc += __shfl_xor(acc, 32, 64);
-	const double a0 = __shfl(acc, 0, 64), a1 = __shfl(acc, 1, 64), a2 = __shfl(acc, 2, 64), a3 = __shfl(acc, 3, 64);
-	if (sub == 0) {
-		const double* d = inv + (size_t)row*16 + 4*r;
-		y[4*(size_t)row + r] = d[0]*a0 + d[1]*a1 + d[2]*a2 + d[3]*a3;
-	}
+	total = WaveSumT(total);
+	if (lane == 0) lds[wave] = total;
+	__syncthreads();
+	if (threadIdx.x == 0) partial[blockIdx.x] = lds[0] + lds[1] + lds[2] + lds[3];
 }
 
-// Deterministic pseudo-random start vector in [-1, 1).
-__global__ void HashVectorKernel(long long n, double* __restrict__ v)
+// Deterministic pseudo-random start vector in [-1, 1), and per workgroup the sum of its squares.
+__global__ void __launch_bounds__(256) HashVectorKernel(long long n, double* __restrict__ v, double* __restrict__ partial)
 {
+	__shared__ double lds[4];
+	double total = 0.0;
 	for (long long i = blockIdx.x*(long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x*blockDim.x) {
 		unsigned long long z = (unsigned long long)i*0x9e3779b97f4a7c15ULL + 0x632be59bd9b4e019ULL;
 		z = (z ^ (z >> 30))*0xbf58476d1ce4e5b9ULL;
 		z = (z ^ (z >> 27))*0x94d049bb133111ebULL;
 		z ^= z >> 31;
-		v[i] = (double)(z >> 11)*(2.0/9007199254740992.0) - 1.0;
+		const double h = (double)(z >> 11)*(2.0/9007199254740992.0) - 1.0;
+		v[i] = h;
+		total += h*h;
 	}
+	total = WaveSumT(total);
+	if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = total;
+	__syncthreads();
+	if (threadIdx.x == 0) partial[blockIdx.x] = lds[0] + lds[1] + lds[2] + lds[3];
+}
+
+// *out = sum of partial[0 .. count), one workgroup
+__global__ void __launch_bounds__(256) SumKernel(const double* __restrict__ partial, int count, double* __restrict__ out)
+{
+	__shared__ double lds[4];
+	double total = 0.0;
+	for (int i = threadIdx.x; i < count; i += 256) total += partial[i];
+	total = WaveSumT(total);
+	if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = total;
+	__syncthreads();
+	if (threadIdx.x == 0) *out = lds[0] + lds[1] + lds[2] + lds[3];
 }
 
 // One colour of a block Gauss-Seidel sweep, in place: for the rows of this
@@ -694,6 +722,8 @@ struct Amg::Impl {
 	DevBuf<float> dinv32;
 	DevBuf<int> status, pivot, step;
 	DevBuf<int> scale_flags;  // per level: S did not fit FP16
+	DevBuf<unsigned int> singular_blocks;        // diagonal blocks without an inverse (counted, not used)
+	DevBuf<double> power[2], power_partial, squares;  // power iteration; per level ||D^-1 A x||^2 of its last step
 
 	void Symbolic(const double* fine_values);
 	void Numeric(const double* fine_values64, const float* fine_values32);
@@ -998,6 +1028,10 @@ void Amg::Impl::Symbolic(const double* fine_values)
 	else dinv64.Allocate(ctx, (size_t)nc*nc);
 	status.Allocate(ctx, 1);
 	scale_flags.Allocate(ctx, L.size());
+	singular_blocks.Allocate(ctx, 1);
+	power_partial.Allocate(ctx, kPowerBlocks);
+	squares.Allocate(ctx, L.size());
+	Fill(ctx, squares.data(), 0.0, static_cast<long long>(L.size()));
 	built = true;
 }
 
@@ -1024,7 +1058,7 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 	}
 	for (size_t l = 0; l < L.size(); ++l) {
 		Level& v = *L[l];
-		BlockInverse64(ctx, v.view(), v.vals64, v.inv64.data());
+		LaunchBlockInverse64(ctx, v.view(), v.vals64, v.inv64.data(), singular_blocks.data());
 		if (precision == TFI_MIXED) {
 			hipLaunchKernelGGL(BlockInverseT32Kernel, dim3(256), dim3(256), 0, ctx->stream, 16LL*v.rows,
 				v.inv64.data(), v.inv32.data());
@@ -1037,53 +1071,54 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 			}
 		}
 	}
-	// FP16 copies of D^-1 A for the Chebyshev levels of the mixed path
-	bool any_scaled = false;
-	for (size_t l = 0; l < L.size(); ++l) any_scaled |= L[l]->s16.size() > 0 && !L[l]->gs;
-	if (any_scaled) {
-		FillInt(ctx, scale_flags.data(), 0, static_cast<long long>(L.size()));
-		for (size_t l = 0; l < L.size(); ++l) {
-			Level& v = *L[l];
-			if (!(v.s16.size() > 0 && !v.gs)) continue;
-			hipLaunchKernelGGL(ScaleBlocksKernel, dim3((v.rows + 3)/4), dim3(256), 0, ctx->stream, v.rows, v.ro,
-				v.diag, v.vals64, v.inv64.data(), v.s16.data(), v.dblock32.data(), scale_flags.data() + l);
-			TFI_LAUNCH_CHECK("ScaleBlocksKernel");
-		}
-		std::vector<int> flags(L.size(), 0);
-		scale_flags.Download(flags.data(), flags.size());
-		for (size_t l = 0; l < L.size(); ++l) L[l]->scaled = L[l]->s16.size() > 0 && !L[l]->gs && flags[l] == 0;
-	}
-	// FP32 A P, or S P where the level's steps read S
+	// FP16 copies of D^-1 A (and S P) for the Chebyshev levels of the mixed path,
+	// FP32 A P for its other levels
+	FillInt(ctx, scale_flags.data(), 0, static_cast<long long>(L.size()));
+	auto wide_ap = [&](Level& v) {
+		hipLaunchKernelGGL(ToFloatKernel2, dim3(Grid(std::min<long long>(v.ap_nnzb*16, 1LL << 22))), dim3(256), 0,
+			ctx->stream, v.ap_nnzb*16, v.ap64.data(), v.ap32.data());
+		TFI_LAUNCH_CHECK("ToFloatKernel2");
+	};
 	if (precision == TFI_MIXED)
 		for (size_t l = 0; l + 1 < L.size(); ++l) {
 			Level& v = *L[l];
-			if (v.scaled)
-				hipLaunchKernelGGL(ScaledGalerkinKernel, dim3(Grid(v.ap_nnzb*16)), dim3(256), 0, ctx->stream, v.ap_nnzb,
-					v.ap_off.data(), v.ap_list.data(), v.s16.data(), v.ap32.data());
-			else if (!v.gs)
-				hipLaunchKernelGGL(ToFloatKernel2, dim3(Grid(std::min<long long>(v.ap_nnzb*16, 1LL << 22))), dim3(256), 0,
-					ctx->stream, v.ap_nnzb*16, v.ap64.data(), v.ap32.data());
-			TFI_LAUNCH_CHECK("FP32 A P");
-		}
-	// lambda_max(D^-1 A) of every Jacobi-smoothed level by power iteration (FP64)
-	for (size_t l = 0; l + 1 < L.size(); ++l) {
-			Level& v = *L[l];
 			if (v.gs) continue;
-			const long long n = 4LL*v.rows;
-			DevBuf<double> a(ctx, n), b(ctx, n);
-			hipLaunchKernelGGL(HashVectorKernel, dim3(Grid(n)), dim3(256), 0, ctx->stream, n, a.data());
-			double lam = 1.0;
-			for (int it = 0; it < kPowerIterations; ++it) {
-				const double nrm = Norm2(ctx, a.data(), n);
-				Scale(ctx, 1.0/nrm, a.data(), n);
-				hipLaunchKernelGGL(DinvAKernel, dim3((v.rows + 3)/4), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols,
-					v.vals64, v.inv64.data(), a.data(), b.data());
-				TFI_LAUNCH_CHECK("DinvAKernel");
-				lam = Norm2(ctx, b.data(), n);
-				std::swap(a, b);
+			if (!v.s16.size()) {
+				wide_ap(v);
+				continue;
 			}
-			v.lambda_max = lam > 0.0 ? lam : 1.0;
+			hipLaunchKernelGGL(ScaleBlocksKernel, dim3((v.rows + 3)/4), dim3(256), 0, ctx->stream, v.rows, v.ro,
+				v.diag, v.vals64, v.inv64.data(), v.s16.data(), v.dblock32.data(), scale_flags.data() + l);
+			TFI_LAUNCH_CHECK("ScaleBlocksKernel");
+			hipLaunchKernelGGL(ScaledGalerkinKernel, dim3(Grid(v.ap_nnzb*16)), dim3(256), 0, ctx->stream, v.ap_nnzb,
+				v.ap_off.data(), v.ap_list.data(), v.s16.data(), v.ap32.data());
+			TFI_LAUNCH_CHECK("ScaledGalerkinKernel");
 		}
+	// lambda_max(D^-1 A) of every Jacobi-smoothed level by power iteration (FP64):
+	// squares[l] = ||D^-1 A x||^2 of the last step's normalised x
+	for (size_t l = 0; l + 1 < L.size(); ++l) {
+		Level& v = *L[l];
+		if (v.gs) continue;
+		const long long n = 4LL*v.rows;
+		if (!power[0].size())  // the first such level is the largest
+			for (auto& p : power) p.Allocate(ctx, n);
+		double* sq = squares.data() + l;
+		const int start = std::min(Grid(n), kPowerBlocks), blocks = std::min((v.rows + 3)/4, kPowerBlocks);
+		auto sum = [&](int count) {
+			hipLaunchKernelGGL(SumKernel, dim3(1), dim3(256), 0, ctx->stream, power_partial.data(), count, sq);
+			TFI_LAUNCH_CHECK("SumKernel");
+		};
+		hipLaunchKernelGGL(HashVectorKernel, dim3(start), dim3(256), 0, ctx->stream, n, power[0].data(),
+			power_partial.data());
+		TFI_LAUNCH_CHECK("HashVectorKernel");
+		sum(start);
+		for (int it = 0; it < kPowerIterations; ++it) {
+			hipLaunchKernelGGL(DinvAKernel, dim3(blocks), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols, v.vals64,
+				v.inv64.data(), power[it & 1].data(), sq, power[(it + 1) & 1].data(), power_partial.data());
+			TFI_LAUNCH_CHECK("DinvAKernel");
+			sum(blocks);
+		}
+	}
 	// coarsest dense inverse, built and inverted on the device
 	Level& c = *L.back();
 	Fill(ctx, dense[0].data(), 0.0, (long long)nc*nc);
@@ -1104,9 +1139,22 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 		matrix = dense[flip].data();
 	}
 	TFI_LAUNCH_CHECK("PanelUpdateKernel");
+	// what the host needs of all this, after one wait
 	int st = 0;
+	std::vector<int> flags(L.size(), 0);
+	std::vector<double> last(L.size(), 0.0);
 	status.Download(&st, 1);
+	scale_flags.Download(flags.data(), flags.size());
+	squares.Download(last.data(), last.size());
 	if (st) throw Error("AMG coarsest operator is singular");
+	for (size_t l = 0; l + 1 < L.size(); ++l) {
+		Level& v = *L[l];
+		v.scaled = v.s16.size() > 0 && !v.gs && flags[l] == 0;
+		if (v.s16.size() > 0 && !v.gs && !v.scaled) wide_ap(v);  // S did not fit FP16
+		if (v.gs) continue;
+		const double lambda = std::sqrt(last[l]);
+		v.lambda_max = lambda > 0.0 ? lambda : 1.0;
+	}
 	if (precision == TFI_MIXED) {
 		hipLaunchKernelGGL(ExtractInverseKernel<float>, dim3(nc), dim3(256), 0, ctx->stream, nc, matrix, pivot.data(),
 			dinv32.data());

@@ -215,13 +215,19 @@ void Residual64(tfi_ctx* ctx, const BsrView& a, const double* values, const doub
 	TFI_LAUNCH_CHECK("BsrSpmvKernel residual");
 }
 
+void LaunchBlockInverse64(tfi_ctx* ctx, const BsrView& a, const double* values, double* inverse,
+	unsigned int* singular)
+{
+	hipLaunchKernelGGL(BlockInverseKernel, dim3((a.rows + 255)/256), dim3(256), 0, ctx->stream, a.rows, a.diagonal,
+		values, inverse, singular);
+	TFI_LAUNCH_CHECK("BlockInverseKernel");
+}
+
 int BlockInverse64(tfi_ctx* ctx, const BsrView& a, const double* values, double* inverse)
 {
 	DevBuf<unsigned int> singular(ctx, 1);
 	Check(hipMemsetAsync(singular.data(), 0, sizeof(unsigned int), ctx->stream), "memset");
-	hipLaunchKernelGGL(BlockInverseKernel, dim3((a.rows + 255)/256), dim3(256), 0, ctx->stream, a.rows, a.diagonal,
-		values, inverse, singular.data());
-	TFI_LAUNCH_CHECK("BlockInverseKernel");
+	LaunchBlockInverse64(ctx, a, values, inverse, singular.data());
 	unsigned int s = 0;
 	singular.Download(&s, 1);
 	return static_cast<int>(s);
