@@ -75,7 +75,8 @@ int tfi_mesh_pattern(tfi_mesh* mesh, int32_t* row_offsets, int32_t* columns, int
 int tfi_mesh_colors(tfi_mesh* mesh, int32_t* element_color);
 /* Basis table: N, grad N and lap N of every (element, quadrature point, basis
  * function), 5 doubles each, evaluated once from the extraction operator and
- * geometry so that every later assembly reads them instead of re-evaluating
+ * geometry so that every later tangent and transport assembly reads them (the
+ * residual takes its fields from the extraction operator) instead of re-evaluating
  * the Bernstein sum-factorisation (the reference evaluates them at every
  * point of every assembly: EvaluateBasisDevice, IgaCudaKernels.cuh:113, called
  * at :303).  enable = 1 builds it, 0 frees it,
