@@ -707,7 +707,8 @@ struct Level {
 	DevBuf<double> inv64;
 	DevBuf<float> vals32_own, inv32;
 	const float* vals32 = nullptr;
-	// mixed precision, Chebyshev levels: S = D^-1 A in FP16 and D in FP32 (scaled: in use)
+	// mixed precision, Chebyshev levels only: S = D^-1 A in FP16 and D in FP32.  scaled: S fits
+	// FP16, the level's steps read it and ap32 holds S P; else they read A and ap32 holds A P
 	DevBuf<_Float16> s16;
 	DevBuf<float> dblock32;
 	bool scaled = false;
@@ -1171,9 +1172,9 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 	if (st) throw Error("AMG coarsest operator is singular");
 	for (size_t l = 0; l + 1 < L.size(); ++l) {
 		Level& v = *L[l];
-		v.scaled = v.s16.size() > 0 && !v.gs && flags[l] == 0;
-		if (v.s16.size() > 0 && !v.gs && !v.scaled) wide_ap(v);  // S did not fit FP16
 		if (v.gs) continue;
+		v.scaled = v.s16.size() > 0 && flags[l] == 0;
+		if (v.s16.size() > 0 && !v.scaled) wide_ap(v);  // S did not fit FP16
 		const double lambda = std::sqrt(last[l]);
 		v.lambda_max = lambda > 0.0 ? lambda : 1.0;
 	}
@@ -1233,7 +1234,7 @@ void Amg::Impl::Cycle(int l, const T* b, T* x)
 			rho = rn;
 			bool done = false;
 			if constexpr (f32) {
-				if (cheb && v.scaled) {
+				if (v.scaled) {
 					hipLaunchKernelGGL(ChebyshevScaledKernel, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols,
 						v.s16.data(), inv, b, static_cast<const float*>(from), to, r, cd, cz);
 					done = true;
@@ -1283,7 +1284,7 @@ void Amg::Impl::Cycle(int l, const T* b, T* x)
 	}
 	bool residual_done = false;
 	if constexpr (f32) {
-		if (cheb && v.scaled) {
+		if (v.scaled) {
 			hipLaunchKernelGGL(ResidualScaledKernel, dim3(grid), dim3(256), 0, ctx->stream, v.rows, v.ro, v.cols,
 				v.s16.data(), inv, v.dblock32.data(), b, static_cast<const float*>(from), r);
 			residual_done = true;
@@ -1311,7 +1312,7 @@ void Amg::Impl::Cycle(int l, const T* b, T* x)
 			hipLaunchKernelGGL(kernel, dim3((v.rows + 7)/8), dim3(256), 0, ctx->stream, v.rows, v.ap_ro.data(), v.ap_cols.data(),
 				static_cast<const T*>(pick(v.ap64, v.ap32)), inv, v.agg.data(), static_cast<const T*>(xc), from, r, first);
 		};
-		if (f32 && cheb && v.scaled) correct(CorrectStepKernel<T, f32>);
+		if (f32 && v.scaled) correct(CorrectStepKernel<T, f32>);
 		else correct(CorrectStepKernel<T, false>);
 		TFI_LAUNCH_CHECK("CorrectStepKernel");
 		more_steps();
@@ -1353,6 +1354,10 @@ void Amg::UseGaussSeidel()
 		Level& v = *I.L[l];
 		v.gs = v.rows >= I.opt.gs_min_rows;
 		if (v.gs && v.color_offsets.empty()) I.Colour(v);
+		// the levels that stay Jacobi-smoothed read A from here on, not S
+		v.s16.Release();
+		v.dblock32.Release();
+		v.scaled = false;
 	}
 }
 
