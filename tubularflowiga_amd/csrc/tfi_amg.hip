@@ -1169,7 +1169,6 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 	status.Download(&st, 1);
 	scale_flags.Download(flags.data(), flags.size());
 	squares.Download(last.data(), last.size());
-	if (st) throw Error("AMG coarsest operator is singular");
 	for (size_t l = 0; l + 1 < L.size(); ++l) {
 		Level& v = *L[l];
 		if (v.gs) continue;
@@ -1178,6 +1177,8 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 		const double lambda = std::sqrt(last[l]);
 		v.lambda_max = lambda > 0.0 ? lambda : 1.0;
 	}
+	// with the levels as their matrices are now: only the coarsest inverse stays the old one
+	if (st) throw Error("AMG coarsest operator is singular");
 	if (precision == TFI_MIXED) {
 		hipLaunchKernelGGL(ExtractInverseKernel<float>, dim3(nc), dim3(256), 0, ctx->stream, nc, matrix, pivot.data(),
 			dinv32.data());
