@@ -63,7 +63,9 @@ typedef struct {
 /* Uploads a FlatMesh (DeviceMesh.hpp:16-68, 70-118), builds the node-block
  * pattern on the GPU (BlockPattern, BlockCsr.hpp:27-55), the element colouring
  * and pair->block map of the deterministic scatter, and the per-quadrature-point
- * geometry (BuildGeometryKernel, IgaCudaKernels.cuh:61-111). */
+ * geometry (BuildGeometryKernel, IgaCudaKernels.cuh:61-111).  Where an
+ * extraction row holds a column more than once, the residual and the tangent
+ * take its last entry. */
 int tfi_mesh_create(tfi_ctx* ctx, int nodes, int elements, const int32_t* element_offsets,
 	const int32_t* connectivity, const int32_t* extraction_offsets, const uint8_t* extraction_columns,
 	const double* extraction_values, const double* bezier_points, tfi_mesh** out);

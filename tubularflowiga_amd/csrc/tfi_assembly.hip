@@ -271,8 +271,9 @@ void SetBasisTable(tfi_mesh* m, int enable)
 	}
 	if (m->basis_table.size() == count) return;
 	m->basis_table.Allocate(ctx, count);
+	const ExtractionRows rows = m->rows();
 	hipLaunchKernelGGL(BasisTableKernel, dim3(m->elements), dim3(256), sizeof(double)*64*m->max_nen, ctx->stream,
-		m->eoff.data(), m->xoff.data(), m->xcol.data(), m->xval.data(), m->geometry.data(), m->basis_table.data());
+		m->eoff.data(), rows.offsets, rows.columns, rows.values, m->geometry.data(), m->basis_table.data());
 	TFI_LAUNCH_CHECK("BasisTableKernel");
 	Sync(ctx);
 }

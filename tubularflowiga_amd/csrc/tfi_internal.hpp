@@ -127,6 +127,12 @@ constexpr int kGeomFields = 20;
 constexpr int kQ = 64;
 constexpr int kMaxBasis = 80;
 
+// Extraction rows as the volume integrals take them: a column at most once per row.
+struct ExtractionRows {
+	const int* offsets;
+	const uint8_t* columns;
+	const double* values;
+};
 }  // namespace tfi
 
 struct tfi_mesh {
@@ -136,6 +142,11 @@ struct tfi_mesh {
 	tfi::DevBuf<int> eoff, conn, xoff;
 	tfi::DevBuf<uint8_t> xcol;
 	tfi::DevBuf<double> xval, bezier;
+	// the extraction rows without the entries that a later one of the same row and column replaces
+	// (allocated only if there are any)
+	tfi::DevBuf<int> unique_xoff;
+	tfi::DevBuf<uint8_t> unique_xcol;
+	tfi::DevBuf<double> unique_xval;
 	// pattern
 	tfi::DevBuf<int> row_offsets, columns, diagonal;
 	long long nnzb = 0;
@@ -170,6 +181,11 @@ struct tfi_mesh {
 	tfi::BsrView view() const
 	{
 		return {nodes, nnzb, row_offsets.data(), columns.data(), diagonal.data()};
+	}
+	tfi::ExtractionRows rows() const
+	{
+		if (unique_xoff.size()) return {unique_xoff.data(), unique_xcol.data(), unique_xval.data()};
+		return {xoff.data(), xcol.data(), xval.data()};
 	}
 };
 

@@ -217,12 +217,49 @@ int NextPow2(int v)
 	return p;
 }
 
+// Extraction rows that repeat a column: in the volume integrals the last entry of
+// a column counts (their kernels spread a row over a dense one, several lanes at
+// once, so each column may be there only once).  The mesh gets a copy of the rows
+// without the entries replaced; most meshes have none, and no copy.
+void UniqueRows(tfi_mesh* m)
+{
+	const int* xoff = m->h_xoff.data();
+	const uint8_t* xcol = m->h_xcol.data();
+	bool repeated = false;
+	for (long long a = 0; a < m->basis_entries && !repeated; ++a) {
+		uint64_t columns = 0;
+		for (int k = xoff[a]; k < xoff[a + 1]; ++k) columns |= 1ull << xcol[k];
+		repeated = __builtin_popcountll(columns) != xoff[a + 1] - xoff[a];
+	}
+	if (!repeated) return;
+	std::vector<int> offsets(1, 0);
+	std::vector<uint8_t> columns;
+	std::vector<double> values;
+	for (long long a = 0; a < m->basis_entries; ++a) {
+		int last[64];
+		for (int k = xoff[a]; k < xoff[a + 1]; ++k) last[xcol[k]] = k;
+		for (int k = xoff[a]; k < xoff[a + 1]; ++k)
+			if (last[xcol[k]] == k) {
+				columns.push_back(xcol[k]);
+				values.push_back(m->h_xval[k]);
+			}
+		offsets.push_back(static_cast<int>(columns.size()));
+	}
+	m->unique_xoff.Allocate(m->ctx, offsets.size());
+	m->unique_xoff.Upload(offsets.data(), offsets.size());
+	m->unique_xcol.Allocate(m->ctx, columns.size());
+	m->unique_xcol.Upload(columns.data(), columns.size());
+	m->unique_xval.Allocate(m->ctx, values.size());
+	m->unique_xval.Upload(values.data(), values.size());
+}
+
 }  // namespace
 
 void BuildMesh(tfi_mesh* m)
 {
 	tfi_ctx* ctx = m->ctx;
 	const int N = m->nodes, E = m->elements;
+	UniqueRows(m);
 	// node -> element adjacency (elements ascending)
 	std::vector<int> n2e_off(N + 1, 0);
 	for (int e = 0; e < E; ++e)

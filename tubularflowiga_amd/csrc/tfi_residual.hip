@@ -46,7 +46,7 @@ constexpr int kFields = 22;  // u (3), p, grad u (9), grad p (3), lap u (3), u_p
 struct ResidualArgs {
 	const int* eoff;
 	const int* conn;
-	const int* xoff;
+	const int* xoff;      // extraction rows, a column at most once per row
 	const uint8_t* xcol;
 	const double* xval;
 	const double* geometry;
@@ -313,7 +313,8 @@ void ElementResiduals(tfi_mesh* m, const double* state, const double* previous, 
 	if (count == 0) return;
 	tfi_ctx* ctx = m->ctx;
 	if (!m->element_rows.size()) m->element_rows.Allocate(ctx, 4*(size_t)m->basis_entries);
-	ResidualArgs a{m->eoff.data(), m->conn.data(), m->xoff.data(), m->xcol.data(), m->xval.data(), m->geometry.data(),
+	const ExtractionRows rows = m->rows();
+	ResidualArgs a{m->eoff.data(), m->conn.data(), rows.offsets, rows.columns, rows.values, m->geometry.data(),
 		state, previous, p.density, p.viscosity, p.dt, m->element_rows.data(), elements, points};
 	const int nen = m->max_nen;
 	const size_t lds = sizeof(double)*(PDoubles(nen) + kQDoubles + 8*(size_t)Rows4(nen) + 48);

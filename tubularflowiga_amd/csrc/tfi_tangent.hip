@@ -68,7 +68,7 @@ typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 struct TangentArgs {
 	const int* eoff;
-	const int* xoff;
+	const int* xoff;         // extraction rows, a column at most once per row
 	const uint8_t* xcol;
 	const double* xval;
 	const double* geometry;
@@ -550,7 +550,8 @@ void AssembleNs(tfi_mesh* m, const double* state, const double* previous, const 
 		m->point_records.Allocate(ctx, (size_t)count*kTangentRec*kQ);
 	}
 	if (!staged) Fill(ctx, jacobian, 0.0, m->nnzb*16);
-	const TangentArgs a{m->eoff.data(), m->xoff.data(), m->xcol.data(), m->xval.data(), m->geometry.data(),
+	const ExtractionRows rows = m->rows();
+	const TangentArgs a{m->eoff.data(), rows.offsets, rows.columns, rows.values, m->geometry.data(),
 		m->point_records.data(), table ? m->basis_table.data() : nullptr, m->pair_offsets.data(), m->pair_block.data(),
 		nullptr, 0, 0, p.density, p.viscosity, p.dt, jacobian, staged ? m->staging.data() : nullptr, m->max_nen};
 	const Inputs in{state, previous, p};
