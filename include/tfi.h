@@ -96,12 +96,18 @@ int tfi_pressure_traction(tfi_mesh* mesh, int count, const int32_t* element, con
 	const double* pressure, double* traction);
 
 /* ------------------------------------------------------------------ kernels (host in/out) */
-/* Negated residual and tangent with a deterministic colour-ordered scatter:
- * tangent TFI_TANGENT_LEGACY = the GPU reference's tau-frozen tangent
+/* Negated residual and tangent, summed in a fixed order (a node's residual in
+ * the order of its elements, a Jacobian block in the order of its elements'
+ * colours): tangent TFI_TANGENT_LEGACY = the GPU reference's tau-frozen tangent
  * (AssembleNavierStokesKernel, IgaCudaKernels.cuh:265-409), TFI_TANGENT_EXACT =
  * the CPU reference's consistent tangent (NavierStokesElement.hpp:244-313).
  * jacobian may be NULL (residual only).  Arrays: state/previous [4N],
- * jacobian [nnzb*16], negative_residual [4N]. */
+ * jacobian [nnzb*16], negative_residual [4N].  The mesh keeps the assembly's
+ * work arrays from its first call to its end: 32 bytes per (element, basis
+ * function), and with a tangent 10.5 KiB per element and the element blocks
+ * (128 bytes per element and pair of functions), or, where these blocks take
+ * more than 4 GiB or a quarter of the memory free at that call, 10.5 KiB per
+ * element of the largest colour alone.  The results are the same either way. */
 int tfi_ns_assemble(tfi_mesh* mesh, const double* state, const double* previous, double density,
 	double viscosity, double dt, double* jacobian, double* negative_residual, int tangent);
 /* y = A x on the mesh pattern (BlockSpmvKernel<4>, SparseKernels.cuh:25-40);

@@ -1,6 +1,8 @@
-"""The tangent added to the Jacobian element colour by element colour: a block is
-the sum of its elements' contributions in the order of their colours, bit for
-bit.  The contributions come from meshes of a single element.  The Jacobian is
+"""The tangent added to the Jacobian element colour by element colour, and the
+one summed from staged element blocks: both leave in a block the sum of its
+elements' contributions in the order of their colours, bit for bit, so which of
+them a mesh takes (its size and the free memory decide) changes no result.  The
+contributions come from meshes of a single element.  By colour the Jacobian is
 read and written plainly, so it may also be in pinned host memory."""
 import ctypes
 import dataclasses
@@ -65,6 +67,20 @@ def _check_rows(ctx, dm, mesh, jac, rows, state, previous):
             blocks = _element_blocks(ctx, mesh, e, state, previous)[np.flatnonzero(nodes == i)[0]]
             want[np.searchsorted(cols[ro[i]:ro[i + 1]], nodes)] += blocks
         assert np.array_equal(jac[ro[i]:ro[i + 1]], want), f"row {i}"
+
+
+@pytest.mark.parametrize("degree", [2, 3])
+def test_staged_sums_in_colour_order(ctx, degree):
+    from tubularflowiga_amd import device
+    mesh = _tube(1, 1, 4, degree)
+    state, previous = _state(mesh.nodes), 0.5 * _state(mesh.nodes)
+    dm = device.DeviceMesh(ctx, mesh)
+    try:
+        jac, _ = dm.assemble(state, previous, RHO, MU, DT)
+        print(f"staged degree={degree} elements={mesh.elements}", flush=True)
+        _check_rows(ctx, dm, mesh, jac, range(0, mesh.nodes, 7), state, previous)
+    finally:
+        dm.close()
 
 
 def test_by_colour_in_device_and_pinned_memory(ctx):

@@ -162,7 +162,7 @@ struct tfi_mesh {
 	// residual rows per entry [basis_entries][4], the node sums' input (allocated by the first assembly)
 	tfi::DevBuf<double> element_rows;
 	// tangent assembly of meshes whose staged element blocks fit: the blocks [element_pairs][16] and, per
-	// pattern block, its (element, a, b) pairs, ascending (allocated by the first tangent assembly)
+	// pattern block, its (element, a, b) pairs by element colour (allocated by the first tangent assembly)
 	int staged = -1;                         // -1: not decided yet
 	tfi::DevBuf<double> staging;
 	tfi::DevBuf<int> block_offsets, block_pairs;

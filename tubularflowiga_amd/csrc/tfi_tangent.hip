@@ -35,10 +35,11 @@
 // fetched while the MFMAs of the slab before run) into LDS, and thread (point,
 // component) forms its coefficients.
 //
-// The blocks leave the workgroup in one of two ways, both of fixed order:
+// The blocks leave the workgroup in one of two ways, which sum in the same order
+// and so to the same bits:
 //   * staged: to a buffer of one block per (element, a, b), all elements in one
-//     launch; a second launch sums each block's contributions in element order
-//     and writes the Jacobian once;
+//     launch; a second launch sums each block's contributions in the order of
+//     the elements' colours and writes the Jacobian once;
 //   * by colour: added to the Jacobian, one launch per element colour (the
 //     elements of a colour share no node).
 //
@@ -381,7 +382,7 @@ __global__ void __launch_bounds__(kThreads, 2) TangentKernel(TangentArgs args)
 	}
 }
 
-// jac[block] = sum of the block's staged contributions, in element order (16 lanes per block)
+// jac[block] = sum of the block's staged contributions, in colour order (16 lanes per block)
 __global__ void __launch_bounds__(kThreads) BlockSumKernel(long long blocks, const int* __restrict__ offsets,
 	const int* __restrict__ pairs, const double* __restrict__ staging, double* __restrict__ jac)
 {
@@ -402,26 +403,16 @@ __global__ void CountPairsKernel(int pairs, const int* __restrict__ pair_block, 
 	if (p < pairs) atomicAdd(count + pair_block[p], 1);
 }
 
-// the pairs of each block, in any order; cursor holds each block's next place
-__global__ void FillPairsKernel(int pairs, const int* __restrict__ pair_block, int* __restrict__ cursor,
+// Appends the pairs of one colour's elements to their blocks' lists; cursor holds each
+// block's next place.  The elements of a colour share no node, so no two threads meet.
+__global__ void __launch_bounds__(kThreads) FillPairsKernel(const int* __restrict__ elements,
+	const long long* __restrict__ pair_offsets, const int* __restrict__ pair_block, int* __restrict__ cursor,
 	int* __restrict__ list)
 {
-	const int p = blockIdx.x*blockDim.x + threadIdx.x;
-	if (p < pairs) list[atomicAdd(cursor + pair_block[p], 1)] = p;
-}
-
-// ascending order within each block's list (short: the elements around two nodes)
-__global__ void SortPairsKernel(long long blocks, const int* __restrict__ offsets, int* __restrict__ list)
-{
-	const long long b = blockIdx.x*(long long)blockDim.x + threadIdx.x;
-	if (b >= blocks) return;
-	const int begin = offsets[b], end = offsets[b + 1];
-	for (int i = begin + 1; i < end; ++i) {
-		const int v = list[i];
-		int j = i;
-		for (; j > begin && list[j - 1] > v; --j) list[j] = list[j - 1];
-		list[j] = v;
-	}
+	const int e = elements[blockIdx.x];
+	const int end = static_cast<int>(pair_offsets[e + 1]);
+	for (int p = static_cast<int>(pair_offsets[e]) + threadIdx.x; p < end; p += kThreads)
+		list[cursor[pair_block[p]]++] = p;
 }
 
 // Staged while the blocks of all elements take at most 4 GiB (46,000 elements of
@@ -431,7 +422,8 @@ __global__ void SortPairsKernel(long long blocks, const int* __restrict__ offset
 // functions 10.0 and 4.3 ms.  The staged blocks cost one more pass over
 // themselves; with 4067 elements per colour (109,824 in all, 10 GB of blocks)
 // the two take the same time (19.9 ms by colour, 20.4 staged), so the memory
-// decides.
+// decides: beside the 4 GiB, a quarter of what is free at the mesh's first
+// tangent assembly.
 constexpr long long kStageBytes = 4LL << 30;
 
 // The staging buffer and the pairs of each block, built by the mesh's first tangent assembly
@@ -453,12 +445,12 @@ void PrepareStaging(tfi_mesh* m)
 	m->block_offsets.Allocate(ctx, m->nnzb + 1);
 	m->block_offsets.Upload(offsets.data(), m->nnzb + 1);
 	m->block_pairs.Allocate(ctx, pairs);
-	hipLaunchKernelGGL(FillPairsKernel, dim3(grid), dim3(kThreads), 0, ctx->stream, pairs, m->pair_block.data(),
-		cursor.data(), m->block_pairs.data());
-	TFI_LAUNCH_CHECK("FillPairsKernel");
-	hipLaunchKernelGGL(SortPairsKernel, dim3(static_cast<unsigned>((m->nnzb + kThreads - 1)/kThreads)), dim3(kThreads), 0,
-		ctx->stream, m->nnzb, m->block_offsets.data(), m->block_pairs.data());
-	TFI_LAUNCH_CHECK("SortPairsKernel");
+	for (int c = 0; c < m->colors; ++c) {
+		hipLaunchKernelGGL(FillPairsKernel, dim3(m->color_offsets[c + 1] - m->color_offsets[c]), dim3(kThreads), 0,
+			ctx->stream, m->color_elements.data() + m->color_offsets[c], m->pair_offsets.data(), m->pair_block.data(),
+			cursor.data(), m->block_pairs.data());
+		TFI_LAUNCH_CHECK("FillPairsKernel");
+	}
 	Sync(ctx);
 	m->staging.Allocate(ctx, 16*(size_t)pairs);
 }
