@@ -280,13 +280,13 @@ void SetBasisTable(tfi_mesh* m, int enable)
 
 // Counted arithmetic of the assembly per element with nen basis functions
 // and Q = 64 points: sum-factorised basis and push-forward (656 + 42 flops per
-// (a, q), none when the basis table supplies them), field interpolation (44),
+// (a, q), none when the basis table supplies them or no tangent asks for them), field interpolation (44),
 // u.grad N and residual row (38), per-point scalars (~300 per q) and the
 // tangent (72 flops per (a, b, q) for the legacy tangent; 132 per (a, b, q)
 // plus ~100 per (a, q) for the exact one).
 double AssemblyFlops(const tfi_mesh* m, bool with_jacobian, bool exact)
 {
-	const double basis = m->basis_table.size() ? 0.0 : 656.0 + 42.0;
+	const double basis = m->basis_table.size() || !with_jacobian ? 0.0 : 656.0 + 42.0;
 	double total = 0.0;
 	for (int e = 0; e < m->elements; ++e) {
 		const double nen = m->h_eoff[e + 1] - m->h_eoff[e];

@@ -218,10 +218,11 @@ class DeviceMesh:
 
     def assembly_flops(self, tangent="exact", with_jacobian=True):
         """Algorithmic flops of one assembly (the library's per-element count:
-        the basis evaluation is not counted when the basis table supplies it)."""
+        the basis evaluation is counted where a tangent has no basis table to
+        take it from)."""
         nen = np.diff(self.host.element_offsets).astype(np.float64)
         pair = (132.0 * nen * nen + 100.0 * nen if tangent == "exact" else 72.0 * nen * nen) if with_jacobian else 0.0
-        basis = 0.0 if self.stats.get("basis_table_bytes", 0) else 656.0 + 42.0
+        basis = 656.0 + 42.0 if with_jacobian and not self.stats.get("basis_table_bytes", 0) else 0.0
         return float(np.sum(64.0 * (nen * (basis + 44.0 + 38.0) + 300.0 + pair)))
 
     def spmv_bytes(self, value_bytes=8):
