@@ -745,7 +745,6 @@ struct Amg::Impl {
 	DevBuf<float> dinv32;
 	DevBuf<int> status, pivot, step;
 	DevBuf<int> scale_flags;  // per level: S did not fit FP16
-	DevBuf<unsigned int> singular_blocks;        // diagonal blocks without an inverse (counted, not used)
 	DevBuf<double> power[2], power_partial, squares;  // power iteration; per level ||D^-1 A x||^2 of its last step
 
 	void Symbolic(const double* fine_values);
@@ -1051,7 +1050,6 @@ void Amg::Impl::Symbolic(const double* fine_values)
 	else dinv64.Allocate(ctx, (size_t)nc*nc);
 	status.Allocate(ctx, 1);
 	scale_flags.Allocate(ctx, L.size());
-	singular_blocks.Allocate(ctx, 1);
 	power_partial.Allocate(ctx, kPowerBlocks);
 	squares.Allocate(ctx, L.size());
 	Fill(ctx, squares.data(), 0.0, static_cast<long long>(L.size()));
@@ -1081,7 +1079,7 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 	}
 	for (size_t l = 0; l < L.size(); ++l) {
 		Level& v = *L[l];
-		LaunchBlockInverse64(ctx, v.view(), v.vals64, v.inv64.data(), singular_blocks.data());
+		LaunchBlockInverse64(ctx, v.view(), v.vals64, v.inv64.data(), nullptr);
 		if (precision == TFI_MIXED) {
 			hipLaunchKernelGGL(BlockInverseT32Kernel, dim3(256), dim3(256), 0, ctx->stream, 16LL*v.rows,
 				v.inv64.data(), v.inv32.data());

@@ -282,7 +282,7 @@ void Spmv64(tfi_ctx* ctx, const BsrView& a, const double* values, const double* 
 void Spmv32(tfi_ctx* ctx, const BsrView& a, const float* values, const double* x, double* y);
 // r = b - A x
 void Residual64(tfi_ctx* ctx, const BsrView& a, const double* values, const double* x, const double* b, double* r);
-// 4x4 inverses of the diagonal blocks; adds the blocks without one to *singular (device).
+// 4x4 inverses of the diagonal blocks; adds the blocks without one to *singular (device, or null).
 void LaunchBlockInverse64(tfi_ctx* ctx, const BsrView& a, const double* values, double* inverse,
 	unsigned int* singular);
 int BlockInverse64(tfi_ctx* ctx, const BsrView& a, const double* values, double* inverse);

@@ -139,7 +139,7 @@ __global__ void BlockInverseKernel(int rows, const int* __restrict__ diag, const
 {
 	const int node = blockIdx.x*blockDim.x + threadIdx.x;
 	if (node >= rows) return;
-	if (InvertDiagonalBlock(node, diag, vals, inv)) atomicAdd(singular, 1u);
+	if (InvertDiagonalBlock(node, diag, vals, inv) && singular) atomicAdd(singular, 1u);
 }
 
 // Same inverse; the singular-block count of each 256-row workgroup goes to
