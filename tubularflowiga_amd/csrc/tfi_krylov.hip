@@ -21,21 +21,23 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kGroup = 8;         // basis vectors of a multi-dot workgroup (one set of wave reductions)
-constexpr int kMaxPer = 8;        // vector entries per thread, at most
+constexpr int kDotPer = 8, kAxpyPer = 4;  // vector entries per thread, at most
+constexpr int kLongPer = 4;       // and of a multi-dot over long vectors
 constexpr int kDotGroups = 2048;  // workgroups of a pass that keep the chip's memory pipes full
 constexpr int kFewBlocks = 32;    // partial sums that the kernel after a multi-dot adds up itself
 
-// Why the split depends on the length: eight entries per thread left 158
-// workgroups for 324,000 entries (25 vectors on average: multi-dot 75 us,
-// multi-axpy 57, 0.9 TB/s) and one for 1800 (20 and 16 us).  With the rule
-// below 13 and 11 us (4.9 TB/s), and 2.8 and 3.9 us; where eight entries per
-// thread already give kDotGroups workgroups nothing changes.
+// Why the split depends on the length: eight entries per thread for any length left
+// 158 workgroups for 324,000 entries (25 vectors on average: multi-dot 75 us,
+// multi-axpy 57, 0.9 TB/s) and one for 1800 (20 and 16 us).  With the rule below
+// 13 and 11 us (4.9 TB/s), and 2.8 and 3.9 us.  The axpy stops at four entries: with
+// eight the loads of eight vectors take 96 registers, and half the waves (8.1
+// million entries, 50 vectors: 797 us, with four entries 567).
 // Entries per thread of a pass over n entries in `lanes` rows of workgroups: as
 // many as leave kDotGroups workgroups (8-byte loads in flight against workgroups
-// to hide their latency), 1 to kMaxPer.
-int EntriesPerThread(long long n, int lanes)
+// to hide their latency), 1 to `most`.
+int EntriesPerThread(long long n, int lanes, int most)
 {
-	int per = kMaxPer;
+	int per = most;
 	while (per > 1 && (n + (long long)kThreads*per - 1)/((long long)kThreads*per)*lanes < kDotGroups) per >>= 1;
 	return per;
 }
@@ -43,10 +45,16 @@ int Blocks(long long n, int per)
 {
 	return static_cast<int>((n + (long long)kThreads*per - 1)/((long long)kThreads*per));
 }
-// Most row blocks EntriesPerThread can ask for: below kDotGroups*2 unless every thread has kMaxPer entries
+// Vectors whose blocks of four entries per thread fill the chip more than twice
+// over: a multi-dot workgroup takes all vectors, w in registers (8.1 million entries,
+// 9 / 25 / 50 vectors: 107 / 282 / 563 us, in rows of eight vectors 132 / 320 / 607;
+// 5 million 66 / 173 / 344 against 78 / 184 / 351, 4.2 million 57 / 154 / 301 against
+// 65 / 150 / 280)
+bool Long(long long n) { return n >= 5000000; }
+// Most row blocks the rules can ask for: below 2*kDotGroups, or with four entries per thread
 int MaxBlocks(long long n)
 {
-	return std::min(Blocks(n, 1), std::max(2*kDotGroups, Blocks(n, kMaxPer)));
+	return std::min(Blocks(n, 1), std::max(2*kDotGroups, Blocks(n, std::min(kAxpyPer, kLongPer))));
 }
 // Vectors too short for a workgroup per CU at one entry per thread: the
 // multi-axpy takes 64 entries per workgroup instead
@@ -108,6 +116,41 @@ __global__ void __launch_bounds__(kThreads) MultiDotKernel(const double* __restr
 	if (threadIdx.x < kGroup && g + (int)threadIdx.x < count) {
 		const int v = threadIdx.x;
 		partial[(long long)(g + v)*gridDim.x + blockIdx.x] = lds[v][0] + lds[v][1] + lds[v][2] + lds[v][3];
+	}
+}
+
+// The same for long vectors (Long): a workgroup takes all vectors, eight at a time,
+// with its part of w in registers.
+__global__ void __launch_bounds__(kThreads) MultiDotLongKernel(const double* __restrict__ V, long long ld, int count,
+	const double* __restrict__ w, long long n, double* __restrict__ partial)
+{
+	constexpr int kPer = kLongPer;
+	__shared__ double lds[kGroup][4];
+	const long long base = (long long)blockIdx.x*kThreads*kPer + threadIdx.x;
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	double wr[kPer];
+#pragma unroll
+	for (int t = 0; t < kPer; ++t) {
+		const long long i = base + (long long)t*kThreads;
+		wr[t] = i < n ? w[i] : 0.0;
+	}
+	for (int g = 0; g < count; g += kGroup) {
+		double acc[kGroup] = {};
+#pragma unroll
+		for (int v = 0; v < kGroup; ++v) {
+			if (g + v >= count) break;
+			const double* Vi = V + (long long)(g + v)*ld;
+#pragma unroll
+			for (int t = 0; t < kPer; ++t) acc[v] += Vi[min(base + (long long)t*kThreads, n - 1)]*wr[t];
+		}
+		const double s = WaveSum8(acc);
+		__syncthreads();  // the sums of the group before have been read
+		if ((lane & 7) == 0) lds[lane >> 3][wave] = s;
+		__syncthreads();
+		if (threadIdx.x < kGroup && g + (int)threadIdx.x < count) {
+			const int v = threadIdx.x;
+			partial[(long long)(g + v)*gridDim.x + blockIdx.x] = lds[v][0] + lds[v][1] + lds[v][2] + lds[v][3];
+		}
 	}
 }
 
@@ -224,16 +267,17 @@ __global__ void NormalizeKernel(const double* __restrict__ src, double* __restri
 int MultiDot(tfi_ctx* ctx, const double* V, long long n, int count, const double* w, double* partial)
 {
 	const int groups = (count + kGroup - 1)/kGroup;
-	const int per = EntriesPerThread(n, groups);
-	const dim3 grid(Blocks(n, per), groups);
-	switch (per) {
-	case 1: hipLaunchKernelGGL(MultiDotKernel<1>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
-	case 2: hipLaunchKernelGGL(MultiDotKernel<2>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
-	case 4: hipLaunchKernelGGL(MultiDotKernel<4>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
-	default: hipLaunchKernelGGL(MultiDotKernel<8>, grid, dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial); break;
-	}
+	const int per = Long(n) ? kLongPer : EntriesPerThread(n, groups, kDotPer);
+	auto launch = [&](auto kernel, int rows) {
+		hipLaunchKernelGGL(kernel, dim3(Blocks(n, per), rows), dim3(kThreads), 0, ctx->stream, V, n, count, w, n, partial);
+	};
+	if (Long(n)) launch(MultiDotLongKernel, 1);
+	else if (per == 1) launch(MultiDotKernel<1>, groups);
+	else if (per == 2) launch(MultiDotKernel<2>, groups);
+	else if (per == 4) launch(MultiDotKernel<4>, groups);
+	else launch(MultiDotKernel<8>, groups);
 	TFI_LAUNCH_CHECK("MultiDotKernel");
-	return static_cast<int>(grid.x);
+	return Blocks(n, per);
 }
 
 // Coefficients from `blocks` partial sums each (0: they are in coef); returns
@@ -253,12 +297,10 @@ int MultiAxpy(tfi_ctx* ctx, const double* V, long long n, int count, double* coe
 		return grid;
 	};
 	if (Short(ctx, n)) return launch(MultiAxpyKernel<1, 4>, ShortBlocks(n));
-	const int per = EntriesPerThread(n, 1);
-	switch (per) {
+	switch (EntriesPerThread(n, 1, kAxpyPer)) {
 	case 1: return launch(MultiAxpyKernel<1, 1>, Blocks(n, 1));
 	case 2: return launch(MultiAxpyKernel<2, 1>, Blocks(n, 2));
-	case 4: return launch(MultiAxpyKernel<4, 1>, Blocks(n, 4));
-	default: return launch(MultiAxpyKernel<8, 1>, Blocks(n, 8));
+	default: return launch(MultiAxpyKernel<4, 1>, Blocks(n, 4));
 	}
 }
 
