@@ -44,7 +44,11 @@ constexpr double kOmegaScale = 1.33;   // block-Jacobi damping = kOmegaScale / l
 constexpr int kPre = 2, kPost = 2;      // Jacobi sweeps / Chebyshev degree
 constexpr double kChebLow = 0.1, kChebHigh = 1.1;  // Chebyshev interval, in units of lambda_max(D^-1 A)
 constexpr int kPowerIterations = 12;
-constexpr int kPowerBlocks = 4096;     // workgroups of a power-iteration product, at most
+// Workgroups of a power-iteration product, at most: a wave with several rows waits for
+// one after the other (16.2 million blocks: 390 us with 4096 workgroups, 368 with
+// 16384, 362 with all 37,554; 230 million 5.6, 5.3 and 5.1 ms), and one workgroup
+// adds up their sums (6 us).
+constexpr int kPowerBlocks = 65536;
 
 template <class T>
 __device__ inline T WaveSumT(T v)
@@ -339,15 +343,21 @@ __global__ void __launch_bounds__(256) HashVectorKernel(long long n, double* __r
 }
 
 // *out = sum of partial[0 .. count), one workgroup
-__global__ void __launch_bounds__(256) SumKernel(const double* __restrict__ partial, int count, double* __restrict__ out)
+constexpr int kSumThreads = 1024;
+__global__ void __launch_bounds__(kSumThreads) SumKernel(const double* __restrict__ partial, int count,
+	double* __restrict__ out)
 {
-	__shared__ double lds[4];
+	__shared__ double lds[kSumThreads/64];
 	double total = 0.0;
-	for (int i = threadIdx.x; i < count; i += 256) total += partial[i];
+#pragma unroll 4
+	for (int i = threadIdx.x; i < count; i += kSumThreads) total += partial[i];
 	total = WaveSumT(total);
 	if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = total;
 	__syncthreads();
-	if (threadIdx.x == 0) *out = lds[0] + lds[1] + lds[2] + lds[3];
+	if (threadIdx.x < 64) {
+		total = WaveSumT(threadIdx.x < kSumThreads/64 ? lds[threadIdx.x] : 0.0);
+		if (threadIdx.x == 0) *out = total;
+	}
 }
 
 // One colour of a block Gauss-Seidel sweep, in place: for the rows of this
@@ -1126,7 +1136,7 @@ void Amg::Impl::Numeric(const double* fine64, const float* fine32)
 		double* sq = squares.data() + l;
 		const int start = std::min(Grid(n), kPowerBlocks), blocks = std::min((v.rows + 3)/4, kPowerBlocks);
 		auto sum = [&](int count) {
-			hipLaunchKernelGGL(SumKernel, dim3(1), dim3(256), 0, ctx->stream, power_partial.data(), count, sq);
+			hipLaunchKernelGGL(SumKernel, dim3(1), dim3(kSumThreads), 0, ctx->stream, power_partial.data(), count, sq);
 			TFI_LAUNCH_CHECK("SumKernel");
 		};
 		hipLaunchKernelGGL(HashVectorKernel, dim3(start), dim3(256), 0, ctx->stream, n, power[0].data(),
