@@ -18,8 +18,9 @@
 // function (K = 4 points), no column is padding, and an accumulator tile holds
 // whole 4x4 blocks: 16 neighbouring lanes hold the 128 contiguous bytes of a
 // block, which go to memory without another transposition.  27 functions take
-// 27 x 2 x 64 = 3456 MFMAs per element (4224 when each component was a 32 x 32
-// product of padded functions), 64 functions 16384 with no padding at all.
+// 28 x 2 x 64 = 3584 MFMAs per element, those of the 28th trial function dropped
+// (4224 when each component was a 32 x 32 product of padded functions), 64
+// functions 16384 with no padding at all.
 // Lane (comp = lane%16, point = lane/16) holds the 12 coefficients of its
 // component at its point for a chunk of four points and forms one B value per
 // MFMA column with three FMAs, used by the kTi test tiles.  FP64 FMAs and FP64
@@ -505,7 +506,7 @@ int LaunchWidth(tfi_mesh* m, const TangentArgs& a, const Inputs& in, bool staged
 template <bool kExact, bool kTable>
 int LaunchClass(tfi_mesh* m, const TangentArgs& a, const Inputs& in, bool staged)
 {
-	// 28 functions: 7 per wave (27, the quadratic spline element, leaves one of 28 idle);
+	// 28 functions: 7 per wave (27, the quadratic spline element, computes one of 28 in vain);
 	// slabs of 16 points while two workgroups' LDS fit a CU, 8 above 32 functions
 	const int nen = m->max_nen;
 	if (nen <= 28) return LaunchWidth<kExact, kTable, 2, 7, 2, 16>(m, a, in, staged);
