@@ -2,8 +2,9 @@
 one summed from staged element blocks: both leave in a block the sum of its
 elements' contributions in the order of their colours, bit for bit, so which of
 them a mesh takes (its size and the free memory decide) changes no result.  The
-contributions come from meshes of a single element.  By colour the Jacobian is
-read and written plainly, so it may also be in pinned host memory."""
+contributions come from meshes of a single element.  By colour the blocks are
+added by atomics in the GPU's own memory, and by loads and stores elsewhere: in
+pinned host memory the same bits come out."""
 import ctypes
 import dataclasses
 

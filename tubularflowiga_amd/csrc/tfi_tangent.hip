@@ -84,6 +84,7 @@ struct TangentArgs {
 	double* jac;
 	double* staging;         // [pair][16], or null: added to jac
 	int max_nen;
+	bool atomic;             // jac is in this GPU's own coarse-grained memory
 };
 
 __host__ __device__ constexpr int PointStride(int nen) { return kRec*nen | 1; }  // odd: points on different banks
@@ -357,30 +358,34 @@ __global__ void __launch_bounds__(kThreads, 2) TangentKernel(TangentArgs args)
 		return;
 	}
 	// Every Jacobian entry receives at most one contribution per launch (the
-	// blocks of one colour are disjoint): a plain read-modify-write, which works
-	// in any memory a kernel can write (FP64 atomics do not in fine-grained host
-	// memory; they took 19.20 ms where this takes 19.26, 109,824 elements of 27
-	// functions).  All slots are asked for together, then the blocks of a trial
-	// function before the first is stored.
-	int slot[kTb][4*kTi];
+	// blocks of one colour are disjoint), so the order of the sums is the order of
+	// the launches.  In the GPU's own memory an atomic leaves the read-modify-write
+	// to the L2, and nothing waits for the old values (1,683,072 elements of 27
+	// functions 267 ms, loaded and stored 273; 109,824 elements 19.18 and 19.26).
+	// Other memory a kernel can write (pinned, managed, another GPU's) does not
+	// carry out FP64 atomics.
+	if (args.atomic) {
+		int slot[kTb][4*kTi];
+#pragma unroll
+		for (int tb = 0; tb < kTb; ++tb)
+#pragma unroll
+			for (int k = 0; k < 4*kTi; ++k)
+				slot[tb][k] = args.pair_block[pbase + min(4*k + kq, nen - 1)*nen + min(bw + tb, nen - 1)];
+#pragma unroll
+		for (int tb = 0; tb < kTb; ++tb)
+#pragma unroll
+			for (int k = 0; k < 4*kTi; ++k)
+				if (4*k + kq < nen && bw + tb < nen)
+					__hip_atomic_fetch_add(args.jac + (size_t)slot[tb][k]*16 + comp, acc[k/4][tb][k%4], __ATOMIC_RELAXED,
+						__HIP_MEMORY_SCOPE_WORKGROUP);
+		return;
+	}
 #pragma unroll
 	for (int tb = 0; tb < kTb; ++tb)
 #pragma unroll
 		for (int k = 0; k < 4*kTi; ++k)
-			slot[tb][k] = args.pair_block[pbase + min(4*k + kq, nen - 1)*nen + min(bw + tb, nen - 1)];
-#pragma unroll
-	for (int tb = 0; tb < kTb; ++tb) {
-		double* at[4*kTi];
-		double old[4*kTi];
-#pragma unroll
-		for (int k = 0; k < 4*kTi; ++k) {
-			at[k] = args.jac + (size_t)slot[tb][k]*16 + comp;
-			old[k] = *at[k];
-		}
-#pragma unroll
-		for (int k = 0; k < 4*kTi; ++k)
-			if (4*k + kq < nen && bw + tb < nen) *at[k] = old[k] + acc[k/4][tb][k%4];
-	}
+			if (4*k + kq < nen && bw + tb < nen)
+				args.jac[(size_t)args.pair_block[pbase + (4*k + kq)*nen + bw + tb]*16 + comp] += acc[k/4][tb][k%4];
 }
 
 // jac[block] = sum of the block's staged contributions, in colour order (16 lanes per block)
@@ -454,6 +459,14 @@ void PrepareStaging(tfi_mesh* m)
 	}
 	Sync(ctx);
 	m->staging.Allocate(ctx, 16*(size_t)pairs);
+}
+
+// Memory of this GPU in which FP64 atomics are carried out: plain device allocations.
+bool OwnMemory(const tfi_ctx* ctx, const void* p)
+{
+	hipPointerAttribute_t a{};
+	Check(hipPointerGetAttributes(&a, p), "hipPointerGetAttributes");
+	return a.type == hipMemoryTypeDevice && !a.isManaged && a.allocationFlags == 0 && a.device == ctx->device;
 }
 
 struct Inputs {
@@ -554,7 +567,8 @@ void AssembleNs(tfi_mesh* m, const double* state, const double* previous, const 
 	const ExtractionRows rows = m->rows();
 	const TangentArgs a{m->eoff.data(), rows.offsets, rows.columns, rows.values, m->geometry.data(),
 		m->point_records.data(), table ? m->basis_table.data() : nullptr, m->pair_offsets.data(), m->pair_block.data(),
-		nullptr, 0, 0, p.density, p.viscosity, p.dt, jacobian, staged ? m->staging.data() : nullptr, m->max_nen};
+		nullptr, 0, 0, p.density, p.viscosity, p.dt, jacobian, staged ? m->staging.data() : nullptr, m->max_nen,
+		!staged && OwnMemory(ctx, jacobian)};
 	const Inputs in{state, previous, p};
 	int launches = 0;
 	if (exact) launches = table ? LaunchClass<true, true>(m, a, in, staged) : LaunchClass<true, false>(m, a, in, staged);
